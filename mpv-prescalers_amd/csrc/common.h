@@ -431,53 +431,74 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 
 // FP32 fast path.  Same quantities through cancellation-free forms (mathematically equal
 // to the reference's): delta = sqrt(((a-d)/2)^2 + b^2) instead of sqrt(T^2/4 - D), and
-// L1 - a = b^2 / ((a-d)/2 + delta) when d < a.  Sets *near when a decision lies within a
-// relative 1e-5 of its bucket boundary, widened for the angle by an FP32 error bound of
-// theta (~16 ulp(T) / (L1 - L2)); exact cases (flat window T = 0, b = 0 exactly) are
-// never near.
+// L1 - a = b^2 / ((a-d)/2 + delta) when d < a.  Square roots and quotients are the
+// hardware's (within 1 ulp), the strength of RULE_LOG2 is the exponent of its argument
+// (floor(log2 v)), and the angle atan2(L1 - a, b) in units of pi/24 is an odd degree-13
+// minimax polynomial of min / max (fitted by the Remez exchange; |error| <= 2.6e-6 units
+// in FP32).  Sets *near, and the caller re-decides in FP64, when a decision lies within a
+// relative 1e-5 of its bucket boundary; for the angle within 3e-5 units (the evaluation's
+// error is below 5e-6) plus the first-order effect 32 u T / (2 delta) of the tensor's own
+// FP32 error (u = 2^-24; 36 terms of five roundings summed one after the other stay below
+// 41 u T / 2 per entry).  Exact cases (flat window T = 0, b = 0 exactly) are never near.
+// Bound by VALU issue: the exactly rounded sqrtf, the library atan2f and log2f that this
+// replaces took about 75 of a hash's ~150 instructions, and an angle margin of 2.4e-4 units
+// sent 3-4x as many sites to FP64.  Measured: ravu-r3 1366x768 44.3 -> 37.5 us, r4-yuv
+// 2 x 1080p 266 -> 248, lite-ar-r3 8 x 1080p 255.6 -> 240.9, 3x-r3 2 x 1080p 54.5 -> 51.6,
+// the same bits out.
 template <int RULE>
 __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* near) {
   const float eps = 1.192092896e-7f;
-  const float pi = 3.141592653589793f;
+  const float rel = 1e-5f, ulp16 = 16.0f * 5.9604645e-8f;
   const float T = a + d;
   const float h = (a - d) * 0.5f;
-  const float delta = sqrtf(h * h + b * b);
-  const float L1 = T * 0.5f + delta;
-  const float L2 = T * 0.5f - delta;
-  // quotients below go through the hardware reciprocal (within 1 ulp of the division):
-  // every decision they feed is re-made in FP64 when it lies within the margins
+  const float delta = __builtin_amdgcn_sqrtf(fmaf(h, h, b * b));
+  const float L1 = fmaf(T, 0.5f, delta);
+  const float L2 = fmaf(T, 0.5f, -delta);
   const float y = h <= 0.f ? delta - h : b * b * __builtin_amdgcn_rcpf(h + delta);  // L1 - a >= 0
-  const float sqrtL1 = sqrtf(L1);
-  const float sqrtL2 = sqrtf(L2);
-  const float at = atan2f(y, b) + pi;
-  float theta = at - pi * floorf(at * (1.0f / 3.141592653589793f));
-  const bool bsmall = fabsf(b) < eps;
-  if (bsmall) theta = 0.f;
+  const float sqrtL1 = __builtin_amdgcn_sqrtf(L1);
+  const float sqrtL2 = __builtin_amdgcn_sqrtf(L2);  // NaN when L2 < 0, as in the reference
+  // u = 24/pi * mod(atan2(y, b) + pi, pi) = 24/pi * atan2(y, b), in [0, 24], since y >= 0 (the wrap at
+  // 24 is a near case); inf/inf counts as 1, a NaN takes angle 0
+  const float ab = fabsf(b);
+  const float r = fminf(fminf(y, ab) * __builtin_amdgcn_rcpf(fmaxf(y, ab)), 1.0f);
+  const float s = r * r;
+  float p = 0.05203826725482941f;
+  p = fmaf(p, s, -0.256717324256897f);
+  p = fmaf(p, s, 0.6082800626754761f);
+  p = fmaf(p, s, -1.0109528303146362f);
+  p = fmaf(p, s, 1.513205647468567f);
+  p = fmaf(p, s, -2.545259475708008f);
+  p = fmaf(p, s, 7.639407634735107f);
+  p *= r;
+  p = y > ab ? 12.0f - p : p;
+  p = b < 0.f ? 24.0f - p : p;
+  const bool bsmall = ab < eps;
+  const float u = bsmall || __builtin_isunordered(y, b) ? 0.f : p;
   const float ssum = sqrtL1 + sqrtL2;
   float mu = (sqrtL1 - sqrtL2) * __builtin_amdgcn_rcpf(ssum);
   if (ssum < eps) mu = 0.f;
-  const float u = theta * static_cast<float>(24.0 / 3.141592653589793);
   Bucket bk;
   bk.angle = static_cast<int>(floorf(u));
-  bk.strength = strength_of<RULE, float>(sqrtL1);
   bk.coherence = mu >= 0.5f ? 2 : (mu >= 0.25f ? 1 : 0);
-  const float rel = 1e-5f, ulp16 = 16.0f * 5.9604645e-8f;
-  bool n = fabsf(fabsf(b) - eps) <= rel * eps + ulp16 * T;
+  bool n = fabsf(ab - eps) <= fmaf(ulp16, T, rel * eps);
   n |= fabsf(L2) <= (rel + ulp16) * T && !(b == 0.f && fminf(a, d) == 0.f);
-  if (!bsmall) {
-    const float cond = (24.0f / pi) * ulp16 * T * __builtin_amdgcn_rcpf(fmaxf(2.0f * delta, 1e-30f));
-    n |= fabsf(u - rintf(u)) <= 24.0f * rel + cond;
-  }
-  if (RULE == RULE_LITE) {
-    n |= fabsf(sqrtL1 - 0.004f) <= rel * 0.004f || fabsf(sqrtL1 - 0.016f) <= rel * 0.016f ||
-         fabsf(sqrtL1 - 0.05f) <= rel * 0.05f;
-  } else if (RULE == RULE_3X) {
-    n |= fabsf(sqrtL1 - 0.005f) <= rel * 0.005f || fabsf(sqrtL1 - 0.02f) <= rel * 0.02f;
+  const float cond = (24.0f / kPiF) * 2.0f * ulp16 * T * __builtin_amdgcn_rcpf(fmaxf(2.0f * delta, 1e-30f));
+  n |= !bsmall && fabsf(u - rintf(u)) <= 3e-5f + cond;
+  if (RULE == RULE_LOG2) {
+    // floor(log2 v) clamped to 0..8; near: v within a relative 6e-5 of 2^1 .. 2^8
+    const float v = fmaf(sqrtL1, 2000.0f, eps);
+    const uint32_t bits = __float_as_uint(v), up = bits + 1024u;
+    bk.strength = v >= 2.0f ? min(static_cast<int>(bits >> 23) - 127, 8) : 0;
+    n |= (up & 0x7fffffu) < 2048u && (up >> 23) - 128u < 8u;
   } else {
-    const float f = log2f(sqrtL1 * 2000.0f + eps);
-    n |= f > 0.5f && f < 8.5f && fabsf(f - rintf(f)) <= rel * 8.0f;
+    bk.strength = strength_of<RULE, float>(sqrtL1);
+    if (RULE == RULE_LITE)
+      n |= fabsf(sqrtL1 - 0.004f) <= rel * 0.004f || fabsf(sqrtL1 - 0.016f) <= rel * 0.016f ||
+           fabsf(sqrtL1 - 0.05f) <= rel * 0.05f;
+    else
+      n |= fabsf(sqrtL1 - 0.005f) <= rel * 0.005f || fabsf(sqrtL1 - 0.02f) <= rel * 0.02f;
   }
-  n |= fabsf(mu - 0.25f) <= rel || fabsf(mu - 0.5f) <= rel;
+  n |= fminf(fabsf(mu - 0.25f), fabsf(mu - 0.5f)) <= rel;
   *near = n && T > 0.f;
   return bk;
 }
