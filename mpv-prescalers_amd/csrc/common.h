@@ -149,83 +149,160 @@ __device__ __forceinline__ float load_elem(const void* p, int64_t idx, int dt, f
   }
 }
 
-// Halo tile of P planes, PH x PW samples each, taken at (ox + col, oy + r) clamped to the
-// W x H plane (clamp-to-edge sampling) and staged to LDS as tile[c][r][col], by NT
-// threads.  `issue` starts every load of the calling thread with no branch on the
-// element type: each sample is fetched as the aligned dword that holds it (which never
-// leaves the sample's own page), its bit offset kept beside it.  `commit` extracts and
-// converts the samples and writes LDS.  A tile therefore costs one memory latency, and a
-// persistent block can issue its next tile while it computes this one.
+// Halo tile of P planes, PH x PW samples each (PW a multiple of 4), taken at (ox + col,
+// oy + r) clamped to the W x H plane (clamp-to-edge sampling) and staged to LDS as
+// tile[c][r][col], by NT threads.  A thread takes items of V = 4 neighbouring samples of a
+// row (2 where items of four would leave half the threads idle and the block waiting for the
+// others): `issue` starts one load per item (V samples at the samples' own alignment),
+// moved inwards where the item reaches past the plane's left or right edge; `commit` converts
+// the samples, repeats the edge ones in such items (tiles at a side edge only) and writes each
+// item to LDS at once.  A tile therefore costs one memory latency, and a persistent block
+// can issue its next tile while it computes this one.  Loads cover exactly V samples of the
+// plane's row: nothing outside the frame is read (planes under V samples wide: sample by
+// sample).
+// Bound by VALU issue: one address and one LDS write per sample took about 19 instructions
+// per sample, 8-17 % of a kernel.  Measured with items: ravu-r4-yuv 2 x 1080p 254.0 -> 240.8
+// us, r3 1366x768 38.1 -> 37.3, nnedi3 nns32 1080p 94.4 -> 93.0 (fewer registers held for
+// the next tile: 123 -> 96 VGPRs, five waves per SIMD), lite and 3x (small tiles) unchanged.
 // Sample addresses are 32-bit element offsets from the frame (plane c * cstride + row *
 // pitch + column, the row term a 24-bit multiply): the host refuses frames that span 2^32
 // elements or more, or whose pitch reaches 2^24 elements (kMaxSpan, kMaxPitch).
-// A pointer into global memory (address space 1): loads through it are global loads, never
+// Pointers into global memory (address space 1): loads through them are global loads, never
 // flat ones (which would also count against the LDS wait counter).
-typedef const __attribute__((address_space(1))) uint32_t* GlobalU32;
+#define MPX_GLOBAL __attribute__((address_space(1)))
+typedef const MPX_GLOBAL uint32_t* GlobalU32;
 
 template <int P, int PH, int PW, int NT>
 struct HaloTile {
-  static constexpr int PN = PH * PW;
-  static constexpr int N = P * PN;
+  static_assert(PW % 4 == 0, "rows are staged in whole items");
+  static constexpr int V = P * PH * PW / 4 * 2 <= NT ? 2 : 4;  // samples per item
+  static constexpr int Q = PW / V;       // items per row
+  static constexpr int N = P * PH * Q;   // items of the tile
   static constexpr int E = (N + NT - 1) / NT;
-  uint32_t v[E];
-  uint32_t sh[E];
+  typedef uint32_t Raw __attribute__((ext_vector_type(V)));  // V dwords, or V samples packed into the first ones
+  typedef float Val __attribute__((ext_vector_type(V)));
+  Raw v[E];
+
+  // samples col .. col + V - 1 of the row at p (LSH: log2 element bytes); W < V: 0 .. W - 1, the last repeated
+  template <int LSH>
+  __device__ __forceinline__ static Raw load(uintptr_t p, int col, int W) {
+    constexpr int D = (V << LSH) / 4;  // dwords of an item (0: two bytes)
+    typedef uint32_t Dwords __attribute__((ext_vector_type(D > 1 ? D : 2)));
+    typedef Dwords DwordsA __attribute__((aligned(1 << LSH)));
+    typedef uint32_t DwordA __attribute__((aligned(1)));
+    typedef uint16_t HalfA __attribute__((aligned(1)));
+    Raw w;
+#pragma unroll
+    for (int k = 0; k < V; ++k) w[k] = 0;
+    if (W >= V) {
+      const uintptr_t a = p + (static_cast<uintptr_t>(static_cast<uint32_t>(col)) << LSH);
+      if constexpr (D > 1) {
+        const Dwords x = *reinterpret_cast<const MPX_GLOBAL DwordsA*>(a);
+#pragma unroll
+        for (int k = 0; k < D; ++k) w[k] = x[k];
+      } else if constexpr (D == 1) {
+        w[0] = *reinterpret_cast<const MPX_GLOBAL DwordA*>(a);
+      } else {
+        w[0] = *reinterpret_cast<const MPX_GLOBAL HalfA*>(a);
+      }
+      return w;
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const uintptr_t a = p + (static_cast<uintptr_t>(static_cast<uint32_t>(min(k, W - 1))) << LSH);
+      if constexpr (LSH == 2) w[k] = *reinterpret_cast<GlobalU32>(a);
+      else if constexpr (LSH == 1) w[k / 2] |= static_cast<uint32_t>(*reinterpret_cast<const MPX_GLOBAL uint16_t*>(a)) << (16 * (k % 2));
+      else w[0] |= static_cast<uint32_t>(*reinterpret_cast<const MPX_GLOBAL uint8_t*>(a)) << (8 * k);
+    }
+    return w;
+  }
+
+  // first sample of the load of the item at column col: its own, moved into the row
+  __device__ __forceinline__ static int load_col(int col, int W) { return max(min(col, W - V), 0); }
+
+  template <int LSH>
+  __device__ __forceinline__ void issue_as(const void* base, int64_t pitch, int64_t cstride, int W, int H, int ox,
+                                           int oy) {
+    const uintptr_t b = reinterpret_cast<uintptr_t>(base);
+    const uint32_t ps = static_cast<uint32_t>(pitch), cs = static_cast<uint32_t>(cstride);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = min(static_cast<int>(threadIdx.x) + e * NT, N - 1);  // tail lanes repeat the last item
+      const int c = P == 1 ? 0 : i / (PH * Q);
+      const int j = i - c * (PH * Q);
+      const int r = j / Q, col = ox + V * (j - r * Q);
+      const int gy = min(max(oy + r, 0), H - 1);
+      const uint32_t off = static_cast<uint32_t>(c) * cs + __umul24(static_cast<uint32_t>(gy), ps);
+      v[e] = load<LSH>(b + (static_cast<uintptr_t>(off) << LSH), load_col(col, W), W);
+    }
+  }
 
   __device__ __forceinline__ void issue(const void* base, int dt, int64_t pitch, int64_t cstride, int W, int H,
                                         int ox, int oy) {
-    const int lsh = dt == DT_F32 ? 2 : (dt == DT_U8 ? 0 : 1);  // log2 element bytes
-    const uintptr_t b = reinterpret_cast<uintptr_t>(base);
-    const uint32_t ps = static_cast<uint32_t>(pitch), cs = static_cast<uint32_t>(cstride);
-    if (ox >= 0 && oy >= 0 && ox + PW <= W && oy + PH <= H) {
-      // interior tile (uniform branch): no clamping, and the per-thread part of each
-      // offset (c*cstride + r*pitch + col) does not depend on the tile
-      const uintptr_t t0 = b + (static_cast<uintptr_t>(__umul24(static_cast<uint32_t>(oy), ps) + ox) << lsh);
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int i = min(static_cast<int>(threadIdx.x) + e * NT, N - 1);
-        const int c = P == 1 ? 0 : i / PN;
-        const int j = i - c * PN;
-        const int r = j / PW, col = j - r * PW;
-        const uint32_t off = static_cast<uint32_t>(c) * cs + __umul24(static_cast<uint32_t>(r), ps) + col;
-        const uintptr_t a = t0 + (static_cast<uintptr_t>(off) << lsh);
-        v[e] = *reinterpret_cast<GlobalU32>(a & ~static_cast<uintptr_t>(3));
-        sh[e] = static_cast<uint32_t>(a & 3) * 8;
-      }
-      return;
-    }
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int i = min(static_cast<int>(threadIdx.x) + e * NT, N - 1);  // tail lanes repeat the last sample
-      const int c = P == 1 ? 0 : i / PN;
-      const int j = i - c * PN;
-      const int r = j / PW, col = j - r * PW;
-      const int gx = min(max(ox + col, 0), W - 1);
-      const int gy = min(max(oy + r, 0), H - 1);
-      const uint32_t off = static_cast<uint32_t>(c) * cs + __umul24(static_cast<uint32_t>(gy), ps) + gx;
-      const uintptr_t a = b + (static_cast<uintptr_t>(off) << lsh);
-      v[e] = *reinterpret_cast<GlobalU32>(a & ~static_cast<uintptr_t>(3));
-      sh[e] = static_cast<uint32_t>(a & 3) * 8;
-    }
+    if (dt == DT_F32) issue_as<2>(base, pitch, cstride, W, H, ox, oy);
+    else if (dt == DT_U8) issue_as<0>(base, pitch, cstride, W, H, ox, oy);
+    else issue_as<1>(base, pitch, cstride, W, H, ox, oy);
   }
+
   // in_rmax = RN(1 / in_max) (from the host): integer samples cost three operations each
-  __device__ __forceinline__ void commit(float* tile, int dt, float in_max, float in_rmax) const {
+  __device__ __forceinline__ static Val convert(Raw w, int dt, float in_max, float in_rmax) {
+    Val f;
+    switch (dt) {
+      case DT_F32:
+#pragma unroll
+        for (int k = 0; k < V; ++k) f[k] = __uint_as_float(w[k]);
+        break;
+      case DT_F16:
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+          f[k] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[k / 2] >> (16 * (k % 2)))));
+        break;
+      case DT_U8:
+#pragma unroll
+        for (int k = 0; k < V; ++k) f[k] = unorm_quotient(static_cast<float>((w[0] >> (8 * k)) & 0xffu), in_max, in_rmax);
+        break;
+      default:
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+          f[k] = unorm_quotient(static_cast<float>((w[k / 2] >> (16 * (k % 2))) & 0xffffu), in_max, in_rmax);
+        break;
+    }
+    return f;
+  }
+
+  // `tile`: 16-byte aligned, P * PH * PW floats; W, ox as issued; `each(i, f)` sees item i's values
+  template <typename Each>
+  __device__ __forceinline__ void commit(float* tile, int dt, float in_max, float in_rmax, int W, int ox,
+                                         Each each) const {
+    const bool whole = ox >= 0 && ox + PW <= W;  // (uniform) every item lies inside its row
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       const int i = static_cast<int>(threadIdx.x) + e * NT;
       if (E * NT == N || i < N) {
-        const uint32_t w = v[e] >> sh[e];
-        float f;
-        switch (dt) {
-          case DT_F32: f = __uint_as_float(v[e]); break;
-          case DT_F16: f = __half2float(__ushort_as_half(static_cast<unsigned short>(w & 0xffffu))); break;
-          case DT_U8: f = unorm_quotient(static_cast<float>(w & 0xffu), in_max, in_rmax); break;
-          default: f = unorm_quotient(static_cast<float>(w & 0xffffu), in_max, in_rmax); break;
+        Val f = convert(v[e], dt, in_max, in_rmax);
+        if (!whole) {
+          // sample k wanted sits at position k + d of the loaded ones, clamped: the edge sample repeats
+          const int col = ox + V * (i % Q), d = col - load_col(col, W);
+          const Val g = f;
+#pragma unroll
+          for (int k = 0; k < V; ++k) {
+            f[k] = g[V - 1];
+#pragma unroll
+            for (int j = V - 2; j >= 0; --j) f[k] = d <= j - k ? g[j] : f[k];
+          }
         }
-        tile[i] = f;
+        reinterpret_cast<Val*>(tile)[i] = f;
+        each(i, f);
       }
     }
   }
+  __device__ __forceinline__ void commit(float* tile, int dt, float in_max, float in_rmax, int W, int ox) const {
+    commit(tile, dt, in_max, in_rmax, W, ox, [](int, const Val&) {});
+  }
 };
+
+// Row length of a staged tile: n samples, rounded up to whole items.
+constexpr int staged_width(int n) { return (n + 3) / 4 * 4; }
 
 __device__ __forceinline__ void store_elem(void* p, int64_t idx, int dt, float v) {
   if (dt == DT_F32)

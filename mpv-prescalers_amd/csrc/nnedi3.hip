@@ -105,7 +105,7 @@ template <int WH, int AXIS, int TY = NY>
 struct Geo {
   static constexpr int K = 8 * WH;
   static constexpr int LO = -(WH / 2 - 1);
-  static constexpr int TW = AXIS == 0 ? NX + 7 : NX + WH - 1;
+  static constexpr int TW = staged_width(AXIS == 0 ? NX + 7 : NX + WH - 1);
   static constexpr int TH = AXIS == 0 ? TY + WH - 1 : TY + 7;
   static constexpr int OX = AXIS == 0 ? -3 : LO;  // tile origin relative to block origin
   static constexpr int OY = AXIS == 0 ? LO : -3;
@@ -223,14 +223,14 @@ template <int WH, int AXIS>
 __global__ __launch_bounds__(256) void nnedi3_valu(NPass p, const float* __restrict__ wt, int nns, int total) {
   using G = Geo<WH, AXIS>;
   constexpr int K = G::K;
-  __shared__ float tile[G::TH * G::TW];
+  __shared__ __attribute__((aligned(16))) float tile[G::TH * G::TW];
   const PassTile pt = pass_tile<NY>(p, xcd_tile(blockIdx.x, total));
   const int f = pt.f;
   const int x0 = pt.x0, y0 = pt.y0;
   {
     NTile<WH, AXIS> ht;
     ht.issue(frame_src(p, f), p.src_dt, pt.sp, 0, pt.W, pt.H, x0 + G::OX, y0 + G::OY);
-    ht.commit(tile, p.src_dt, p.src_max, p.src_rmax);
+    ht.commit(tile, p.src_dt, p.src_max, p.src_rmax, pt.W, x0 + G::OX);
   }
   __syncthreads();
   const int tx = threadIdx.x % NX, ty = threadIdx.x / NX;
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma(NPass p, const void* __res
   // neuron tiles (nns 16 / 32: 2-3 % slower) and less from four on (nns 64: -2 %, nns 256:
   // -1 %).
   constexpr bool LINES = M::FUSED_SCALE && TERMS == 1 && (WH == 6 || NSL * TPW >= 4);
-  __shared__ float tile[2][G::TH * G::TW];
+  __shared__ __attribute__((aligned(16))) float tile[2][G::TH * G::TW];
   __shared__ float2 stab[LINES ? LS::N : 1];   // line statistics of the staged tile
   __shared__ __attribute__((aligned(16))) T xhi[NPX * XS];
   __shared__ __attribute__((aligned(16))) T xlo[M::LO_ROWS ? NPX * XS : 16];
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma(NPass p, const void* __res
     const int y0 = pt.y0, x0 = pt.x0;
     // The other buffer was last read two tiles ago, before the barrier below was last
     // passed by every wave.
-    ht.commit(tile[buf], p.src_dt, p.src_max, p.src_rmax);
+    ht.commit(tile[buf], p.src_dt, p.src_max, p.src_rmax, pt.W, x0 + G::OX);
     __syncthreads();
     if (L + static_cast<int>(gridDim.x) < total_tiles) issue(xcd_tile(L + gridDim.x, total_tiles));
     if constexpr (LINES) {
@@ -798,7 +798,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma32(NPass p, const void* __r
   // keep the per-pixel two-pass variance, good to one).  On 8x4 windows the table's build
   // pass and barrier cost more than the 32-term sums they save (measured 1-3% slower).
   constexpr bool LINES = M::FUSED_SCALE && TERMS == 1 && WH == 6;
-  __shared__ float tile[2][G::TH * G::TW];
+  __shared__ __attribute__((aligned(16))) float tile[2][G::TH * G::TW];
   __shared__ float2 stab[LINES ? LS::N : 1];   // line statistics of the staged tile
   __shared__ __attribute__((aligned(16))) T xhi[NPX * XS];
   __shared__ __attribute__((aligned(16))) T xlo[M::LO_ROWS ? NPX * XS : 8];
@@ -876,7 +876,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma32(NPass p, const void* __r
     const int y0 = pt.y0, x0 = pt.x0;
     // the other buffer was last read two tiles ago, before the barrier below was last
     // passed by every wave
-    ht.commit(tile[buf], p.src_dt, p.src_max, p.src_rmax);
+    ht.commit(tile[buf], p.src_dt, p.src_max, p.src_rmax, pt.W, x0 + G::OX);
     __syncthreads();
     if (L + static_cast<int>(gridDim.x) < total_tiles) issue(xcd_tile(L + gridDim.x, total_tiles));
     if constexpr (LINES) {

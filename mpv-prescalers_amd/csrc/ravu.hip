@@ -34,7 +34,7 @@ __device__ __forceinline__ void stage_planes(float* tile, const void* base, int 
   __builtin_amdgcn_s_setprio(1);  // the loads go out ahead of other waves' arithmetic
   h.issue(base, dt, pitch, cstride, W, H, ox, oy);
   __builtin_amdgcn_s_setprio(0);
-  h.commit(tile, dt, in_max, in_rmax);
+  h.commit(tile, dt, in_max, in_rmax, W, ox);
 }
 
 // Planes staged per tile: the P input planes, plus for rgb a fourth holding the BT.709
@@ -100,10 +100,10 @@ __global__ __launch_bounds__(TX * TY) void ravu_3x_kernel(Io io, const __half* _
   constexpr int P = CH == 0 ? 1 : 3;
   constexpr int N = 2 * R - 1;
   constexpr int HALO = R - 1;
-  constexpr int PW = TX + 2 * HALO, PH = TY + 2 * HALO, PN = PW * PH;
+  constexpr int PW = staged_width(TX + 2 * HALO), PH = TY + 2 * HALO, PN = PW * PH;
   constexpr int C = (N * N - 1) / 2;
   constexpr int NTEX = 2 * (C + 1);
-  __shared__ float tile[staged_planes<CH>() * PN];
+  __shared__ __attribute__((aligned(16))) float tile[staged_planes<CH>() * PN];
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
@@ -259,8 +259,8 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(6))) vo
                                                          int64_t int11_frame, int total) {
   constexpr int P = CH == 0 ? 1 : 3;
   constexpr int N = 2 * R;
-  constexpr int PW = TX + N - 1, PH = TY + N - 1, PN = PW * PH;
-  __shared__ float tile[staged_planes<CH>() * PN];
+  constexpr int PW = staged_width(TX + N - 1), PH = TY + N - 1, PN = PW * PH;
+  __shared__ __attribute__((aligned(16))) float tile[staged_planes<CH>() * PN];
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
@@ -340,9 +340,9 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
                                                            const float* __restrict__ int11, int64_t int11_frame,
                                                            int total) {
   constexpr int P = CH == 0 ? 1 : 3;
-  constexpr int PW = TX + 2 * R + 1, PH = TY + 2 * R + 1, PN = PW * PH;  // offsets -R..R
-  __shared__ float hk[staged_planes<CH>() * PN];   // input (HOOKED)
-  __shared__ float i11[staged_planes<CH>() * PN];  // ravu_int11
+  constexpr int PW = staged_width(TX + 2 * R + 1), PH = TY + 2 * R + 1, PN = PW * PH;  // offsets -R..R
+  __shared__ __attribute__((aligned(16))) float hk[staged_planes<CH>() * PN];   // input (HOOKED)
+  __shared__ __attribute__((aligned(16))) float i11[staged_planes<CH>() * PN];  // ravu_int11
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
@@ -354,8 +354,8 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
     a.issue(in, io.in_dt, ft.in_pitch, ft.in_cstride, ft.W, ft.H, x0 - R, y0 - R);
     b.issue(int11 + f * int11_frame, DT_F32, ft.W, plane, ft.W, ft.H, x0 - R, y0 - R);
     __builtin_amdgcn_s_setprio(0);
-    a.commit(hk, io.in_dt, io.in_max, io.in_rmax);
-    b.commit(i11, DT_F32, 1.f, 1.f);
+    a.commit(hk, io.in_dt, io.in_max, io.in_rmax, ft.W, x0 - R);
+    b.commit(i11, DT_F32, 1.f, 1.f, ft.W, x0 - R);
   }
   __syncthreads();
   if constexpr (CH == 2) {

@@ -20,11 +20,11 @@ __global__ __launch_bounds__(TX * TY) void ravu_lite_kernel(Io io, const __half*
   constexpr int NT = TX * TY;  // threads per block
   constexpr int N = 2 * R - 1;
   constexpr int HALO = R - 1;
-  constexpr int PW = TX + 2 * HALO;
+  constexpr int PW = staged_width(TX + 2 * HALO);
   constexpr int PH = TY + 2 * HALO;
   constexpr int NTEX = (N * N + 1) / 2;
   constexpr int C = (N * N - 1) / 2;
-  __shared__ float tile[PH * PW];
+  __shared__ __attribute__((aligned(16))) float tile[PH * PW];
   // AR: per staged sample (l + 0.1)^32, (1.1 - l)^32 and the ^33 terms, computed once per
   // sample instead of once per pixel whose anti-ringing window reads it (up to 13)
   __shared__ float4 pw[AR ? PH * PW : 1];
@@ -36,23 +36,24 @@ __global__ __launch_bounds__(TX * TY) void ravu_lite_kernel(Io io, const __half*
   const void* in = frame_in(io, frame);
 
   {
-    HaloTile<1, PH, PW, NT> h;
+    typedef HaloTile<1, PH, PW, NT> Tile;
+    Tile h;
     __builtin_amdgcn_s_setprio(1);  // the loads go out ahead of other waves' arithmetic
     h.issue(in, io.in_dt, ft.in_pitch, 0, ft.W, ft.H, x0 - HALO, y0 - HALO);
     __builtin_amdgcn_s_setprio(0);
-    h.commit(tile, io.in_dt, io.in_max, io.in_rmax);
-  }
-  if constexpr (AR) {
-    // each thread takes the samples it staged itself (the commit's index pattern), so the
-    // one block barrier below orders both tables
-    for (int i = threadIdx.x; i < PH * PW; i += NT) {
-      const float l = tile[i];
-      const float p0 = 0.1f + l, m0 = 1.1f - l;
-      float p32 = p0, m32 = m0;
+    // (AR: each thread tabulates the samples it stages, so one block barrier orders both)
+    h.commit(tile, io.in_dt, io.in_max, io.in_rmax, ft.W, x0 - HALO, [&](int i, const typename Tile::Val& f) {
+      if constexpr (AR) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k) { p32 *= p32; m32 *= m32; }
-      pw[i] = make_float4(p32, m32, p32 * p0, m32 * m0);
-    }
+        for (int k = 0; k < Tile::V; ++k) {
+          const float p0 = 0.1f + f[k], m0 = 1.1f - f[k];
+          float p32 = p0, m32 = m0;
+#pragma unroll
+          for (int t = 0; t < 5; ++t) { p32 *= p32; m32 *= m32; }
+          pw[Tile::V * i + k] = make_float4(p32, m32, p32 * p0, m32 * m0);
+        }
+      }
+    });
   }
   __syncthreads();
 
