@@ -2,7 +2,7 @@
 
 Headline workload: nnedi3-nns32-win8x4 luma 2x by two field-doubling passes,
 one 1920x1080 FP16 plane -> 3840x2160, FP16-MFMA form (FP32 accumulation); a step is
-one frame through both passes.  Reported: output Mpixel/s, the plain FP32 VALU form's
+one frame through both passes.  Reported: output Mpixel/s, the FP32-accuracy form's
 Mpixel/s and the ratio, p50/p99 per-frame latency, the dominant kernel's roofline
 (double_x pass: 2*K*2*nns FLOP per predicted pixel, W x 2H predicted pixels per
 launch), secondary variants, the serving loop, and the C FP32 restatement's CPU throughput on
@@ -255,7 +255,7 @@ def serving_bench(duration_s=2.0, rate=2000.0, seed=5):
     native = _native_queue(reqs, prec, total_px, gaps)
     # (c) one frame per launch on one stream: the plain request loop (launch, wait for the
     # result, next request), the same launches issued back to back, and the plain request
-    # loop with the plain forms (FP32 VALU NNEDI3)
+    # loop with every variant at FP32 accuracy
     single_sync = _one_per_launch(pool, reqs, prec, total_px, sync=True)
     single_async = _one_per_launch(pool, reqs, prec, total_px, sync=False)
     plain_sync = _one_per_launch(pool, reqs, {v: "fp32" for v in prec}, total_px, sync=True)

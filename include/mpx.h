@@ -36,7 +36,7 @@ extern "C" {
 #define MPX_F32 3
 
 /* ---- NNEDI3 contraction precision (RAVU always computes in FP32) ------------------ */
-#define MPX_PREC_FP32 0   /* plain FP32 VALU kernel                                       */
+#define MPX_PREC_FP32 0   /* FP32 accuracy: operands as high + low FP16 parts on MFMA     */
 #define MPX_PREC_FP16 1   /* FP16 MFMA, one product, FP32 accumulation                    */
 #define MPX_PREC_BF16 2   /* BF16 MFMA, high/low split (three products), FP32 accumulation */
 #define MPX_PREC_FP8 3    /* FP8 e4m3 MFMA, per-neuron power-of-two scales, FP32 accum.   */

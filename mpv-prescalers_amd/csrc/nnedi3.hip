@@ -13,16 +13,21 @@
 // is taken as mean((x-m)^2) (two passes), the same value as the reference's
 // E[x^2]-m^2 without its FP32 cancellation.
 //
-// Two forms:
-//  * nnedi3_valu: plain FP32, one thread per pixel, weights read as wave-uniform scalars.
-//  * nnedi3_mfma / nnedi3_mfma32: the [neurons x K] x [K x pixels] contraction on MFMA
-//    (v_mfma_f32_16x16x32_{f16,bf16}, K = 48 as two 32-chunks, zero padded; or
-//    v_mfma_f32_32x32x16_{f16,bf16}, K = 48 as three 16-chunks), FP32
-//    accumulation, with the biases as the accumulator's initial value; weights and inputs
-//    optionally split into high+low 16-bit parts (three products) so the contraction
-//    keeps ~22 (FP16) / ~16 (BF16) bits.  The exp2 /
-//    reciprocal / blend epilogue stays FP32.  Persistent blocks keep their neuron slice's
-//    weights in VGPRs for the whole launch.
+// nnedi3_mfma / nnedi3_mfma32: the [neurons x K] x [K x pixels] contraction on MFMA
+// (v_mfma_f32_16x16x32_{f16,bf16}, K = 48 as two 32-chunks, zero padded; or
+// v_mfma_f32_32x32x16_{f16,bf16}, K = 48 as three 16-chunks), FP32 accumulation, with the
+// biases as the accumulator's initial value; weights and inputs optionally split into
+// high+low 16-bit parts (three products) so the contraction keeps ~22 (FP16) / ~16 (BF16)
+// bits.  The exp2 / reciprocal / blend epilogue stays FP32.  Persistent blocks keep their
+// neuron slice's weights in VGPRs for the whole launch.
+//
+// MPX_PREC_FP32 is the FP16 split form with both operands scaled by 2^12: the products it
+// drops (low x low) and the parts' own rounding are about 2^-23 of |w||x'|, below what K
+// FP32 multiply-adds in a row round away.  Against 64-bit arithmetic its relative error is
+// 0.6-0.9e-7 over the ten networks (8-bit codes and floats), where the one-thread-per-pixel
+// FP32 kernel that it replaces had 1.0-1.6e-7; that kernel was bound by its multiply-adds
+// on the VALU (6,953 instructions per pixel for nns64 win8x6, matrix cores idle):
+// nns64-win8x6 1280x720 520.9 -> 139.5 us.
 #include "common.h"
 #include "launch.h"
 #include "nnedi3.h"
@@ -121,19 +126,26 @@ using NTile = HaloTile<1, Geo<WH, AXIS, TY>::TH, Geo<WH, AXIS, TY>::TW, 256>;
 // mean, 1/std (0 below the variance threshold) and std of a K-sample window held in
 // registers; the window is replaced by its centred form, and by its centred, normalised
 // form when SCALE (otherwise the caller applies 1/std, e.g. inside its 16-bit conversion).
-template <int K, bool SCALE = true>
+// PARTS = 8 (the split forms): both sums run as eight partial sums combined in a tree, which
+// keeps their rounding error near an ulp (the mean's goes straight into the result); the
+// 16-bit forms, which cannot resolve that, take one running sum (0.6 % faster at nns32).
+template <int K, bool SCALE = true, int PARTS = 1>
 __device__ __forceinline__ void normalise(float* x, float& m, float& sd, float& is) {
-  float sum = x[0];
+  auto total = [](const float* p) {
+    if constexpr (PARTS == 1) return p[0];
+    else return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+  };
+  constexpr int L = K / PARTS;  // samples per partial sum
+  float part[PARTS];
 #pragma unroll
-  for (int k = 1; k < K; ++k) sum += x[k];
-  m = sum * (1.0f / static_cast<float>(K));
-  float ss = 0.f;
+  for (int k = 0; k < K; ++k) part[k / L] = k % L ? part[k / L] + x[k] : x[k];
+  m = total(part) * (1.0f / static_cast<float>(K));
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     x[k] -= m;
-    ss += x[k] * x[k];
+    part[k / L] = k % L ? fmaf(x[k], x[k], part[k / L]) : x[k] * x[k];
   }
-  const float v = ss * (1.0f / static_cast<float>(K));
+  const float v = total(part) * (1.0f / static_cast<float>(K));
   // hardware reciprocal square root (within 1 ulp); the threshold test is exact
   is = v >= kVarEps ? __builtin_amdgcn_rsqf(v) : 0.f;
   sd = v * is;
@@ -215,51 +227,6 @@ __device__ __forceinline__ const void* frame_src(const NPass& p, int f) {
 __device__ __forceinline__ void* frame_dst(const NPass& p, int f) {
   if (p.ntab_dst) return p.tab_dst[f];
   return static_cast<char*>(p.dst) + static_cast<int64_t>(f) * p.dst_bstride * elem_bytes(p.dst_dt);
-}
-
-// ----------------------------------------------------------------------------- FP32 VALU
-
-template <int WH, int AXIS>
-__global__ __launch_bounds__(256) void nnedi3_valu(NPass p, const float* __restrict__ wt, int nns, int total) {
-  using G = Geo<WH, AXIS>;
-  constexpr int K = G::K;
-  __shared__ __attribute__((aligned(16))) float tile[G::TH * G::TW];
-  const PassTile pt = pass_tile<NY>(p, xcd_tile(blockIdx.x, total));
-  const int f = pt.f;
-  const int x0 = pt.x0, y0 = pt.y0;
-  {
-    NTile<WH, AXIS> ht;
-    ht.issue(frame_src(p, f), p.src_dt, pt.sp, 0, pt.W, pt.H, x0 + G::OX, y0 + G::OY);
-    ht.commit(tile, p.src_dt, p.src_max, p.src_rmax, pt.W, x0 + G::OX);
-  }
-  __syncthreads();
-  const int tx = threadIdx.x % NX, ty = threadIdx.x / NX;
-  const int x = x0 + tx, y = y0 + ty;
-  if (x >= pt.W || y >= pt.H) return;
-  float xv[K];
-#pragma unroll
-  for (int a = 0; a < 8; ++a)
-#pragma unroll
-    for (int b = 0; b < WH; ++b) xv[a * WH + b] = tile[G::at(tx, ty, a, b)];
-  float m, sd;
-  float is;
-  normalise<K>(xv, m, sd, is);
-  float wsum = 0.f, vsum = 0.f;
-  for (int n = 0; n < nns; ++n) {
-    const float* w = wt + n * (2 * K + 2);
-    float s1 = w[2 * K], s2 = w[2 * K + 1];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      s1 = fmaf(w[k], xv[k], s1);
-      s2 = fmaf(w[K + k], xv[k], s2);
-    }
-    const float e = __builtin_amdgcn_exp2f(s1);
-    const float q = s2 * __builtin_amdgcn_rcpf(1.0f + fabsf(s2));
-    wsum += e;
-    vsum = fmaf(e, q, vsum);
-  }
-  const float pred = fminf(fmaxf(m + 5.0f * vsum * __builtin_amdgcn_rcpf(wsum) * sd, 0.f), 1.f);
-  store_result<AXIS>(p, frame_dst(p, f), pt.dp, x, y, tile[G::centre(tx, ty)], pred);
 }
 
 // ----------------------------------------------------------------------------- MFMA
@@ -653,7 +620,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma(NPass p, const void* __res
           sd = v * is;
         } else {
           // two-pass: the window comes back centred (FUSED_SCALE) or normalised
-          normalise<K, !M::FUSED_SCALE>(xv, m, sd, is);
+          normalise<K, !M::FUSED_SCALE, M::FUSED_SCALE || FORM == F_FP8 ? 1 : 8>(xv, m, sd, is);
         }
         M::write_row(xhi + threadIdx.x * XS, xlo + (M::LO_ROWS ? threadIdx.x * XS : 0), xv, LINES ? m : 0.f,
                      (LINES || M::FUSED_SCALE) ? is : 1.f, xscale, SCALED);
@@ -906,7 +873,7 @@ __global__ __launch_bounds__(256, 2) void nnedi3_mfma32(NPass p, const void* __r
           sd = v * is;
         } else {
           // two-pass: the window comes back centred (FUSED_SCALE) or normalised
-          normalise<K, !M::FUSED_SCALE>(xv, m, sd, is);
+          normalise<K, !M::FUSED_SCALE, M::FUSED_SCALE || FORM == F_FP8 ? 1 : 8>(xv, m, sd, is);
         }
         M::write_row(xhi + threadIdx.x * XS, xlo + (M::LO_ROWS ? threadIdx.x * XS : 0), xv, LINES ? m : 0.f,
                      (LINES || M::FUSED_SCALE) ? is : 1.f, xscale, SCALED);
@@ -981,11 +948,6 @@ static hipError_t run_pass(const NnediWeights& nw, NPass& p, hipStream_t st, hip
     for (int f = 0; f < p.ntab_src; ++f) p.tiles[f + 1] = p.tiles[f] + ((p.fW[f] + NX - 1) / NX) * ((p.fH[f] + ty - 1) / ty);
     return p.tiles[p.ntab_src];
   };
-  if (nw.precision == 0) {
-    const int tiles = count_tiles(NY);
-    return launch_done(nnedi3_valu<WH, AXIS>, dim3(tiles), dim3(256), st, done, p, static_cast<const float*>(nw.w),
-                       nw.nns, tiles);
-  }
   int total = 0;                         // tiles of the launched MFMA instance (launch_inst)
   hipError_t le = hipErrorInvalidValue;  // the MFMA launch's status
   const int nt = nw.nns / 16;

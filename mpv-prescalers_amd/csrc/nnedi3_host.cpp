@@ -60,13 +60,16 @@ int nnedi3_prepare(mpx_ctx* ctx, int nns, int wh, int precision, NnediWeights* o
     return fail(MPX_ERR_IO, "unexpected shape of " + name);
   out->nns = nns;
   out->wh = wh;
+  // MPX_PREC_FP32 runs the FP16 split form, whose products keep FP32's accuracy: see nnedi3.hip
+  if (precision == MPX_PREC_FP32) precision = MPX_PREC_FP16X3;
   out->precision = precision;
-  // The FP16 split form carries power-of-two operand scales (window x256, weights x256)
-  // so that the low parts stay normal FP16 numbers (MFMA flushes FP16 subnormal inputs);
-  // BF16 has FP32's exponent range, the single-product FP16 form has no low parts.
+  // The FP16 split form carries power-of-two operand scales (window x4096, |x'| <= 6.9;
+  // weights x4096, |w| <= 6.8 over the shipped networks) so that the low parts stay normal
+  // FP16 numbers (MFMA flushes FP16 subnormal inputs); BF16 has FP32's exponent range, the
+  // single-product FP16 form has no low parts.
   const bool f16 = precision == MPX_PREC_FP16 || precision == MPX_PREC_FP16X3;
-  out->xscale = precision == MPX_PREC_FP16X3 ? 256.f : 1.f;
-  out->wscale = precision == MPX_PREC_FP16X3 ? 256.f : 1.f;
+  out->xscale = precision == MPX_PREC_FP16X3 ? 4096.f : 1.f;
+  out->wscale = precision == MPX_PREC_FP16X3 ? 4096.f : 1.f;
   const double ws = out->wscale, accs = static_cast<double>(out->xscale) * out->wscale;
   auto W1 = [&](int n, int k) { return static_cast<double>(t[n * (2 * K + 2) + k]) * kLog2e; };
   auto W2 = [&](int n, int k) { return static_cast<double>(t[n * (2 * K + 2) + K + k]); };
@@ -74,28 +77,11 @@ int nnedi3_prepare(mpx_ctx* ctx, int nns, int wh, int precision, NnediWeights* o
   auto B2 = [&](int n) { return static_cast<double>(t[n * (2 * K + 2) + 2 * K + 1]); };
 
   std::vector<float> bias(2 * nns);
-  const double bscale = precision == MPX_PREC_FP32 ? 1.0 : accs;
   for (int n = 0; n < nns; ++n) {
-    bias[2 * n] = static_cast<float>(B1(n) * bscale);
-    bias[2 * n + 1] = static_cast<float>(B2(n) * bscale);
+    bias[2 * n] = static_cast<float>(B1(n) * accs);
+    bias[2 * n + 1] = static_cast<float>(B2(n) * accs);
   }
   const void* p = nullptr;
-  if (precision == MPX_PREC_FP32) {
-    std::vector<float> w(static_cast<size_t>(nns) * (2 * K + 2));
-    for (int n = 0; n < nns; ++n) {
-      float* r = &w[static_cast<size_t>(n) * (2 * K + 2)];
-      for (int k = 0; k < K; ++k) {
-        r[k] = static_cast<float>(W1(n, k));
-        r[K + k] = static_cast<float>(W2(n, k));
-      }
-      r[2 * K] = bias[2 * n];
-      r[2 * K + 1] = bias[2 * n + 1];
-    }
-    rc = ctx->upload(name + "/fp32", w.data(), w.size() * 4, &p);
-    if (rc) return rc;
-    out->w = p;
-    return MPX_OK;
-  }
   rc = ctx->upload(name + "/bias_x" + std::to_string(static_cast<long long>(accs)), bias.data(), bias.size() * 4, &p);
   if (rc) return rc;
   out->bias = static_cast<const float*>(p);
