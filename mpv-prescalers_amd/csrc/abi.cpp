@@ -318,8 +318,8 @@ int mpx_plan_create(mpx_ctx* ctx, const char* name, int in_w, int in_h, int targ
         rc = ctx->lut16("ravu_3x_lut" + r, &p->lut, nullptr);
         break;
       case MPX_FAMILY_RAVU_ZOOM:
-        rc = ctx->lut16("ravu_zoom_lut" + r, &p->lut, nullptr);
-        if (!rc && v->ar) rc = ctx->lut16("ravu_zoom_lut" + r + "_ar", &p->lut_ar, nullptr);
+        rc = ctx->lut16("ravu_zoom_lut" + r, &p->lut, nullptr, true);
+        if (!rc && v->ar) rc = ctx->lut16("ravu_zoom_lut" + r + "_ar", &p->lut_ar, nullptr, true);
         if (!rc) rc = mpx::zoom_plan_create(ctx, p.get(), in_w, in_h, p->info.out_w, p->info.out_h);
         break;
       case MPX_FAMILY_NNEDI3:

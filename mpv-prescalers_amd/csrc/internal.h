@@ -124,7 +124,9 @@ struct mpx_ctx {
   }
 
   // FP16 copy (RNE, as the rgba16f upload) of a LUT weight file, resident on the device.
-  int lut16(const std::string& name, const __half** out, std::vector<uint32_t>* shape) {
+  // zoom: rows hold texel groups of 9 phases, 9 g + x; they are uploaded phase by phase,
+  // x * groups + g, so that all groups of two neighbouring phases lie side by side.
+  int lut16(const std::string& name, const __half** out, std::vector<uint32_t>* shape, bool zoom = false) {
     std::lock_guard<std::mutex> lk(mu);
     auto it = weights.find(name);
     if (it == weights.end()) {
@@ -132,7 +134,12 @@ struct mpx_ctx {
       std::vector<uint32_t> d;
       if (int rc = mpx_host::load_table(wdir, name, data, d)) return rc;
       std::vector<_Float16> h(data.size());
-      for (size_t i = 0; i < data.size(); ++i) h[i] = static_cast<_Float16>(data[i]);
+      const size_t row = zoom ? d[1] * size_t{4} : data.size(), groups = row / 36;
+      for (size_t i = 0; i < data.size(); ++i) {
+        const size_t c = i % row, texel = c / 4;
+        const size_t at = zoom ? i - c + 4 * (texel % 9 * groups + texel / 9) + c % 4 : i;
+        h[at] = static_cast<_Float16>(data[i]);
+      }
       void* p = nullptr;
       int rc = alloc(h.size() * 2, &p);
       if (rc) return rc;
