@@ -451,6 +451,14 @@ __device__ __forceinline__ void structure_tensor(Get get, T& a, T& b, T& d) {
   }
 }
 
+// Gradient grid of an N x N window: positions P0 .. P1 - 1 on both axes.
+template <int N>
+struct GradGrid {
+  static constexpr int P0 = N <= 4 ? 0 : 1;
+  static constexpr int P1 = N <= 4 ? N : N - 1;
+  static constexpr int M = P1 - P0;
+};
+
 enum Rule : int { RULE_LITE = 0, RULE_3X = 1, RULE_LOG2 = 2 };
 
 template <int RULE> struct RuleInfo;
@@ -512,11 +520,13 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 // hardware's (within 1 ulp), the strength of RULE_LOG2 is the exponent of its argument
 // (floor(log2 v)), and the angle atan2(L1 - a, b) in units of pi/24 is an odd degree-13
 // minimax polynomial of min / max (fitted by the Remez exchange; |error| <= 2.6e-6 units
-// in FP32).  Sets *near, and the caller re-decides in FP64, when a decision lies within a
-// relative 1e-5 of its bucket boundary; for the angle within 3e-5 units (the evaluation's
-// error is below 5e-6) plus the first-order effect 32 u T / (2 delta) of the tensor's own
-// FP32 error (u = 2^-24; 36 terms of five roundings summed one after the other stay below
-// 41 u T / 2 per entry).  Exact cases (flat window T = 0, b = 0 exactly) are never near.
+// in FP32).  Sets *near, and the caller re-decides in FP64, when a decision may differ from
+// the exact one.  The tensor's own FP32 error (u = 2^-24): 36 terms of five roundings summed
+// one after the other give a, d within 41 u of themselves and b within 41 u T / 2, hence
+// sqrt(L1) within a relative 41 u = 2.5e-6 (margin 3.8e-6), L2 within 41 u T (6.9e-6 T), mu
+// within 55 u at 1/4 and 92 u at 1/2 (6e-6), and the angle within 29 u T / (2 delta) (32 u,
+// plus 1e-5 units for the evaluation, whose error is below 5e-6).  Exact cases (flat window
+// T = 0, b = 0 exactly) are never near.
 // Bound by VALU issue: the exactly rounded sqrtf, the library atan2f and log2f that this
 // replaces took about 75 of a hash's ~150 instructions, and an angle margin of 2.4e-4 units
 // sent 3-4x as many sites to FP64.  Measured: ravu-r3 1366x768 44.3 -> 37.5 us, r4-yuv
@@ -525,7 +535,7 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 template <int RULE>
 __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* near) {
   const float eps = 1.192092896e-7f;
-  const float rel = 1e-5f, ulp16 = 16.0f * 5.9604645e-8f;
+  const float rel = 4e-6f, u24 = 24.0f * 5.9604645e-8f;
   const float T = a + d;
   const float h = (a - d) * 0.5f;
   const float delta = __builtin_amdgcn_sqrtf(fmaf(h, h, b * b));
@@ -557,16 +567,16 @@ __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* nea
   Bucket bk;
   bk.angle = static_cast<int>(floorf(u));
   bk.coherence = mu >= 0.5f ? 2 : (mu >= 0.25f ? 1 : 0);
-  bool n = fabsf(ab - eps) <= fmaf(ulp16, T, rel * eps);
-  n |= fabsf(L2) <= (rel + ulp16) * T && !(b == 0.f && fminf(a, d) == 0.f);
-  const float cond = (24.0f / kPiF) * 2.0f * ulp16 * T * __builtin_amdgcn_rcpf(fmaxf(2.0f * delta, 1e-30f));
-  n |= !bsmall && fabsf(u - rintf(u)) <= 3e-5f + cond;
+  bool n = fabsf(ab - eps) <= fmaf(u24, T, rel * eps);
+  n |= fabsf(L2) <= (rel + 2.0f * u24) * T && !(b == 0.f && fminf(a, d) == 0.f);
+  const float cond = (24.0f / kPiF) * 32.0f * 5.9604645e-8f * T * __builtin_amdgcn_rcpf(fmaxf(2.0f * delta, 1e-30f));
+  n |= !bsmall && fabsf(u - rintf(u)) <= 1e-5f + cond;
   if (RULE == RULE_LOG2) {
-    // floor(log2 v) clamped to 0..8; near: v within a relative 6e-5 of 2^1 .. 2^8
+    // floor(log2 v) clamped to 0..8; near: v within a relative 3.8e-6 (7.6e-6) below (above) 2^1 .. 2^8
     const float v = fmaf(sqrtL1, 2000.0f, eps);
-    const uint32_t bits = __float_as_uint(v), up = bits + 1024u;
+    const uint32_t bits = __float_as_uint(v), up = bits + 64u;
     bk.strength = v >= 2.0f ? min(static_cast<int>(bits >> 23) - 127, 8) : 0;
-    n |= (up & 0x7fffffu) < 2048u && (up >> 23) - 128u < 8u;
+    n |= (up & 0x7fffffu) < 128u && (up >> 23) - 128u < 8u;
   } else {
     bk.strength = strength_of<RULE, float>(sqrtL1);
     if (RULE == RULE_LITE)
@@ -575,7 +585,7 @@ __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* nea
     else
       n |= fabsf(sqrtL1 - 0.005f) <= rel * 0.005f || fabsf(sqrtL1 - 0.02f) <= rel * 0.02f;
   }
-  n |= fminf(fabsf(mu - 0.25f), fabsf(mu - 0.5f)) <= rel;
+  n |= fminf(fabsf(mu - 0.25f), fabsf(mu - 0.5f)) <= 6e-6f;
   *near = n && T > 0.f;
   return bk;
 }
@@ -588,6 +598,89 @@ __device__ __forceinline__ int bucket_row(Bucket bk, int rows) {
   int row = (bk.angle * RuleInfo<RULE>::S + bk.strength) * 3 + bk.coherence;
   return min(max(row, 0), rows - 1);
 }
+
+// hash_reference out of line: its registers (the double atan2 alone takes 56) would set the
+// occupancy of every wave.
+template <int RULE>
+__device__ __attribute__((noinline)) Bucket hash_fp64(double a, double b, double d) {
+  return hash_reference<RULE, double>(a, b, d);
+}
+
+// The structure tensor of the sites of this wave whose bit is set in `mask`, in FP64 and in
+// the oracle's operation order (no contraction): the whole wave works on one site at a time, a
+// grid point per lane (at most 36), and the points' terms are then added in grid order.
+// `at(site)` gives an accessor (X, Y) -> sample of the window of lane `site`.  Every lane of
+// the wave must be active.  a, b, d are set in the lanes of `mask`.
+// Bound by the latency of the wave that takes it, which holds its block's LDS meanwhile: one
+// lane's serial evaluation (up to 36 points of two five-point derivatives, r4 rgb luma in FP64
+// per sample) took 10-20 us where a wave otherwise lives about 10 (ravu-r4-rgb 640x360 51.6 us,
+// 21.2 with the path switched off; with the shared one 28.7).  It also costs the kernel fewer
+// registers: zoom-ar-r2-rgb 96 VGPRs and scratch -> 81 and none, 4 x 720p -> 1440p 340.4 ->
+// 288.9 us.  Small central-difference windows (lite, 3x) keep a lane's own evaluation: several
+// of their lanes are near at once (lite-r2 8 x 1080p 126 us, shared 150).
+template <int N, bool FIVE, typename At>
+__device__ __forceinline__ void wave_tensor(uint64_t mask, At at, double& a, double& b, double& d) {
+#pragma clang fp contract(off)
+  using GG = GradGrid<N>;
+  constexpr int POINTS = GG::M * GG::M;
+  const int lane = threadIdx.x & 63;
+  const int pt = min(lane, POINTS - 1);
+  const int X = GG::P0 + pt / GG::M, Y = GG::P0 + pt % GG::M;
+  const double w = gauss_w<N>(pt);
+  // one derivative: position p of the line s, forward/backward at the border (its two samples
+  // clamped into the window), central or five-point inside
+  auto derivative = [](auto s, int p) {
+#pragma clang fp contract(off)
+    const double lo = s(max(p - 1, 0)), hi = s(min(p + 1, N - 1));
+    const double diff = hi - lo;
+    double r = p == 0 || p == N - 1 ? diff : diff / 2.0;
+    if constexpr (FIVE && N >= 5) {
+      const double num = -s(min(p + 2, N - 1)) + 8.0 * hi - 8.0 * lo + s(max(p - 2, 0));
+      if (p >= 2 && p + 2 <= N - 1) r = div_const(num, 12.0, 1.0 / 12.0);
+    }
+    return r;
+  };
+  auto lane_value = [](double v, int i) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(u), i);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(u >> 32), i);
+    return __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo));
+  };
+  while (mask) {
+    const int site = __builtin_ctzll(mask);
+    mask &= mask - 1;
+    const auto sample = at(site);
+    const double gx = derivative([&](int k) { return sample(k, Y); }, X);
+    const double gy = derivative([&](int k) { return sample(X, k); }, Y);
+    const double ta = gx * gx * w, tb = gx * gy * w, td = gy * gy * w;
+    double sa = 0.0, sb = 0.0, sd = 0.0;
+#pragma unroll 4
+    for (int i = 0; i < POINTS; ++i) {
+      sa = sa + lane_value(ta, i);
+      sb = sb + lane_value(tb, i);
+      sd = sd + lane_value(td, i);
+    }
+    if (lane == site) {
+      a = sa;
+      b = sb;
+      d = sd;
+    }
+  }
+}
+
+// The FP64 re-decision of the lanes whose FP32 decision is near a boundary (see wave_tensor).
+template <int N, bool FIVE, int RULE, typename At>
+__device__ __forceinline__ void redecide(bool near, At at, Bucket& bk) {
+  const uint64_t mask = __ballot(near);
+  if (mask) {
+    double a = 0.0, b = 0.0, d = 0.0;
+    wave_tensor<N, FIVE>(mask, at, a, b, d);
+    if (near) bk = hash_fp64<RULE>(a, b, d);
+  }
+}
+
+// Value of lane `i` (uniform) in every lane.
+__device__ __forceinline__ int from_lane(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
 
 // Hash of one site: FP32, re-decided in FP64 when near a boundary.  getf(i) -> float
 // and getd(i) -> double return window sample i (getd widens the same stored values, and
@@ -603,6 +696,20 @@ __device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
     structure_tensor<N, FIVE, double, LEAN>(getd, ad, bd, dd);
     bk = hash_reference<RULE, double>(ad, bd, dd);
   }
+  return bk;
+}
+
+// The same with the wave's shared re-decision (wave_tensor).  getf(i) returns
+// window sample i; at(site): see wave_tensor.  All lanes of the wave call it together; lanes
+// without a site (`valid` false) read their window too (inside the staged tile) but are never
+// re-decided.
+template <int N, bool FIVE, int RULE, bool LEAN, typename GetF, typename At>
+__device__ __forceinline__ Bucket ravu_hash_wave(bool valid, GetF getf, At at) {
+  float a, b, d;
+  structure_tensor<N, FIVE, float, LEAN>(getf, a, b, d);
+  bool near = false;
+  Bucket bk = hash_fast<RULE>(a, b, d, &near);
+  redecide<N, FIVE, RULE>(near && valid, at, bk);
   return bk;
 }
 

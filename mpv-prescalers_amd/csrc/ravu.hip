@@ -71,12 +71,19 @@ __device__ __forceinline__ double luma_d(const float* t, int o, int n) {
   return static_cast<double>(t[o]);
 }
 
+// Whether full RAVU re-decides a wave's near sites together (wave_tensor) or each lane its own:
+// together for r3 and r4 and where a sample is the FP64 luma of three (r3 luma 1366x768 37.2 ->
+// 33.4 us, r3 rgb 2 x 1080p 174.5 -> 153.5, r4 rgb 640x360 51.6 -> 28.6, r2 rgb 135.5 -> 117.5);
+// r2's 16 points are soon done, and several of its lanes are near at once (r2 luma together:
+// 99.1 -> 131.9).
+template <int N, int CH>
+constexpr bool wave_redecide() { return N >= 6 || CH == 2; }
+
 // Hash of the site whose N x N window starts at staged-tile offset o (sample i at
 // o + (i % N) * PW + i / N), with the FP64 re-decision out of line: it is rare, and inlined
 // its registers (the double atan2 alone takes 56) would set the occupancy of every wave
-// (r4 rgb step1: 96 -> 51 VGPRs).  Its register budget follows its callers' (the kernel asks
-// for 6 waves per SIMD), so it takes the lean tensor form to stay out of scratch.  Used
-// where it pays (full-RAVU step1); ravu-3x measured 2-3 % slower with it.
+// (r2 luma step1).  Its register budget follows its callers' (the kernel asks
+// for 6 waves per SIMD), so it takes the lean tensor form to stay out of scratch.
 template <int N, bool FIVE, int RULE, int CH, int PW, int PN>
 __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o) {
   double a, b, d;
@@ -84,13 +91,22 @@ __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o)
                                           d);
   return hash_reference<RULE, double>(a, b, d);
 }
-template <int N, bool FIVE, int RULE, int CH, int PW, int PN, bool LEAN>
-__device__ __forceinline__ Bucket hash_site(const float* t, int o) {
-  float a, b, d;
-  structure_tensor<N, FIVE, float, LEAN>([&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); }, a, b, d);
-  bool near = false;
-  const Bucket bk = hash_fast<RULE>(a, b, d, &near);
-  return near ? redecide_site<N, FIVE, RULE, CH, PW, PN>(t, o) : bk;
+// Hash of this lane's step-1 site; all lanes of the wave together.
+template <int N, int CH, int PW, int PN>
+__device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
+  auto sample = [&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); };
+  if constexpr (wave_redecide<N, CH>()) {
+    return ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
+      const float* w = t + from_lane(o, site);
+      return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
+    });
+  } else {
+    float a, b, d;
+    structure_tensor<N, true, float, true>(sample, a, b, d);
+    bool near = false;
+    const Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
+    return near && valid ? redecide_site<N, true, RULE_LOG2, CH, PW, PN>(t, o) : bk;
+  }
 }
 
 // ----------------------------------------------------------------------------- RAVU-3x
@@ -274,9 +290,10 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(6))) vo
   }
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   const int x = x0 + tx, y = y0 + ty;
-  if (x >= ft.W || y >= ft.H) return;
+  const bool valid = x < ft.W && y < ft.H;
   auto off = [&](int i) { return (ty + i % N) * PW + tx + i / N; };
-  const Bucket bk = hash_site<N, true, RULE_LOG2, CH, PW, PN, true>(tile, off(0));
+  const Bucket bk = hash_site<N, CH, PW, PN>(tile, off(0), valid);
+  if (!valid) return;
   const int row = bucket_row<RULE_LOG2>(bk, 648);
   if (io.buckets) io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y) * ft.W + x] = row;
   float res[P];
@@ -303,7 +320,7 @@ __device__ __host__ constexpr int lat2y(int X, int Y) { return STEP == 2 ? Y - X
 template <int R, int CH, int STEP, int PW, int PN>
 __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restrict__ lut, const float* hk,
                                              const float* i11, int base, const FrameTile& ft, int x, int y,
-                                             int64_t plane) {
+                                             bool valid, int64_t plane) {
   constexpr int P = CH == 0 ? 1 : 3;
   constexpr int N = 2 * R;
   auto src = [&](int i) -> const float* {
@@ -311,8 +328,20 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
     const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
     return (px & 1) ? i11 + base + ((py - 1) >> 1) * PW + ((px - 1) >> 1) : hk + base + (py >> 1) * PW + (px >> 1);
   };
-  const Bucket bk = ravu_hash<N, true, RULE_LOG2, true>([&](int i) { return luma_f<CH>(src(i), 0, PN); },
-                                                  [&](int i) { return luma_d<CH>(src(i), 0, PN); });
+  auto sample = [&](int i) { return luma_f<CH>(src(i), 0, PN); };
+  Bucket bk;
+  if constexpr (wave_redecide<N, CH>()) {
+    bk = ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
+      const int o = from_lane(base, site);
+      return [hk, o](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
+        const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
+        return luma_d<CH>(hk, o + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
+      };
+    });
+  } else {
+    bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return luma_d<CH>(src(i), 0, PN); });
+  }
+  if (!valid) return;
   const int row = bucket_row<RULE_LOG2>(bk, 648);
   if (io.buckets)
     io.buckets[ft.f * io.bucket_bstride + (STEP - 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row;
@@ -341,8 +370,8 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
                                                            int total) {
   constexpr int P = CH == 0 ? 1 : 3;
   constexpr int PW = staged_width(TX + 2 * R + 1), PH = TY + 2 * R + 1, PN = PW * PH;  // offsets -R..R
-  __shared__ __attribute__((aligned(16))) float hk[staged_planes<CH>() * PN];   // input (HOOKED)
-  __shared__ __attribute__((aligned(16))) float i11[staged_planes<CH>() * PN];  // ravu_int11
+  __shared__ __attribute__((aligned(16))) float tiles[2][staged_planes<CH>() * PN];
+  float *hk = tiles[0], *i11 = tiles[1];  // input (HOOKED), ravu_int11
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
@@ -365,11 +394,11 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
   }
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   const int x = x0 + tx, y = y0 + ty;
-  if (x >= ft.W || y >= ft.H) return;
+  const bool valid = x < ft.W && y < ft.H;
   const int base = (ty + R) * PW + tx + R;  // LDS offset of (x, y)
-  lattice_site<R, CH, 2, PW, PN>(io, lut, hk, i11, base, ft, x, y, plane);
+  lattice_site<R, CH, 2, PW, PN>(io, lut, hk, i11, base, ft, x, y, valid, plane);
   __builtin_amdgcn_sched_barrier(0);
-  lattice_site<R, CH, 3, PW, PN>(io, lut, hk, i11, base, ft, x, y, plane);
+  lattice_site<R, CH, 3, PW, PN>(io, lut, hk, i11, base, ft, x, y, valid, plane);
 }
 
 template <int T>

@@ -243,9 +243,8 @@ __global__ __launch_bounds__(256) void zoom_phase_kernel(int4* tab, int in_w, in
 
 // One block per TX x TY output tile, one thread per output pixel (kZoomTiles).  (Kernels
 // without anti-ringing: at least 6 waves per SIMD, a register budget their out-of-line
-// re-decision inherits; r2 anti-ringing kernels and r3 ones on 16 x 16 tiles: 5, 96 VGPRs
-// with a few bytes of scratch, measured 1-8 % faster than 4 waves at 118-126.)  TAB: the plan has the pre-interpolated
-// weight table; separate instances keep the per-pixel bilinear fetch's registers out of the
+// re-decision inherits; r2 anti-ringing kernels and r3 ones on 16 x 16 tiles: 5, at most 96
+// VGPRs, measured 1-8 % faster than 4 waves.)  TAB: the plan has the pre-interpolated weight table; separate instances keep the per-pixel bilinear fetch's registers out of the
 // table path.
 template <int R, bool AR, int CH, bool TAB, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((R == 2 || TX == 16) ? 5 : 1) : 6))) void ravu_zoom_kernel(Io io, const __half* __restrict__ lut,
@@ -280,23 +279,29 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   __syncthreads();
   // hash every base pixel the tile's outputs use (unclamped LUT row: bucket 9-row blocks
   // are clamped per texel by the bilinear fetch, as the sampler does)
-  for (int i = threadIdx.x; i < nbx * nby; i += blockDim.x) {
+  // (whole waves: the re-decision takes all lanes; those past the last base pixel repeat it)
+  for (int i0 = threadIdx.x & ~63; i0 < nbx * nby; i0 += TX * TY) {
+    const int lane_i = i0 + static_cast<int>(threadIdx.x & 63), i = min(lane_i, nbx * nby - 1);
     const int by = i / nbx, bx = i - by * nbx;
     auto off = [&](int s) { return (by + s % N) * PW + bx + s / N; };
-    if constexpr (AR) {
-      // the anti-ringing tap loop sets these kernels' register count: the re-decision stays
-      // inline, in the lean tensor forms for r3 (r3 rgb: 216 -> 123 VGPRs)
-      const Bucket bk = ravu_hash<N, true, RULE_LITE, (R >= 3)>([&](int s) { return zluma_f<CH>(tile, off(s), PN); },
-                                                      [&](int s) { return zluma_d<CH>(tile, off(s), PN); });
-      bucket[by * BX + bx] = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
+    auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
+    int value;
+    if constexpr (R >= 3 || AR || CH == 2) {
+      const int origin = by * PW + bx;
+      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, (R >= 3)>(lane_i == i, sample, [&](int site) {
+        const float* t = tile + from_lane(origin, site);
+        return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
+      });
+      value = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
     } else {
       float ta, tb, td;
-      structure_tensor<N, true, float, (R >= 3)>([&](int s) { return zluma_f<CH>(tile, off(s), PN); }, ta, tb, td);
+      structure_tensor<N, true, float, false>(sample, ta, tb, td);
       bool near = false;
       const Bucket bk = hash_fast<RULE_LITE>(ta, tb, td, &near);
-      bucket[by * BX + bx] = near ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
-                                    : (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
+      value = near && lane_i == i ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
+                                  : (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
     }
+    if (lane_i == i) bucket[by * BX + bx] = value;
   }
   __syncthreads();
 
