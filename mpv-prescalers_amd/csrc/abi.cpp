@@ -688,7 +688,7 @@ static mpx::TileShape tile_shape(const mpx_plan* plan, int t) {
   switch (plan->v->family) {
     case MPX_FAMILY_RAVU_LITE: return mpx::kLiteTiles[t];
     case MPX_FAMILY_RAVU_3X: return mpx::k3xTiles[t];
-    case MPX_FAMILY_RAVU: return mpx::kRavuTiles[t];
+    case MPX_FAMILY_RAVU: return mpx::kRavuTiles[mpx::ravu_tile_index(plan->v->radius, plan->v->channels, t)];
     case MPX_FAMILY_RAVU_ZOOM: return mpx::kZoomTiles[t];
     default: return mpx::TileShape{0, 0};
   }

@@ -51,6 +51,15 @@ constexpr TileShape kLiteTiles[] = {{64, 4}, {32, 8}, {32, 4}};
 constexpr TileShape k3xTiles[] = {{32, 8}, {64, 4}};
 constexpr TileShape kRavuTiles[] = {{32, 8}, {32, 16}, {64, 8}};
 constexpr TileShape kZoomTiles[] = {{32, 8}, {16, 16}};
+// Full RAVU r3 has its shapes in another order, its fastest first: 64 x 8 for luma and yuv (r3
+// 1366x768 32.0 us, 32 x 8 34.8, 32 x 16 33.9; 4 x 1080p 159.4, 162.3, 163.7), 32 x 16 for rgb, whose
+// fourth plane of 64 x 8 tiles leaves two blocks per compute unit (2 x 1080p 140.4 us, 32 x 8
+// 150.5, 64 x 8 169.5).  r4 is faster on 32 x 8 (r4-yuv 195.9 us, 205.9, 204.8).
+constexpr int ravu_tile_index(int r, int channels, int tile) {
+  if (r != 3) return tile;
+  if (channels == 2) return tile < 2 ? 1 - tile : tile;
+  return (tile + 2) % 3;
+}
 constexpr int kLiteTileCount = sizeof(kLiteTiles) / sizeof(kLiteTiles[0]);
 constexpr int k3xTileCount = sizeof(k3xTiles) / sizeof(k3xTiles[0]);
 constexpr int kRavuTileCount = sizeof(kRavuTiles) / sizeof(kRavuTiles[0]);

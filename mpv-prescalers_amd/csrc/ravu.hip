@@ -19,10 +19,8 @@
 namespace mpx {
 
 // Tiles: TX x TY pixels per block of TX * TY threads, one input pixel (3x) or site (full
-// RAVU) per thread, from the families' shape lists (k3xTiles, kRavuTiles).  Full RAVU's halo
-// is up to 9 rows, so its tiles are taller than 3x's: 32 x 8 by default (r4 lattice: 41 x 17
-// staged samples per 256 sites, against 73 x 13 for a 64 x 4 tile), 32 x 16 and 64 x 8 on
-// 512 threads as alternatives.
+// RAVU; two in the pair form of step 1) per thread, from the families' shape lists (k3xTiles,
+// kRavuTiles).  Full RAVU's halo is up to 9 rows, so its tiles are taller than 3x's.
 
 
 // Stage P planes of a frame into LDS: tile[c][r][col] = plane c at
@@ -71,13 +69,12 @@ __device__ __forceinline__ double luma_d(const float* t, int o, int n) {
   return static_cast<double>(t[o]);
 }
 
-// Whether full RAVU re-decides a wave's near sites together (wave_tensor) or each lane its own:
-// together for r3 and r4 and where a sample is the FP64 luma of three (r3 luma 1366x768 37.2 ->
-// 33.4 us, r3 rgb 2 x 1080p 174.5 -> 153.5, r4 rgb 640x360 51.6 -> 28.6, r2 rgb 135.5 -> 117.5);
-// r2's 16 points are soon done, and several of its lanes are near at once (r2 luma together:
-// 99.1 -> 131.9).
-template <int N, int CH>
-constexpr bool wave_redecide() { return N >= 6 || CH == 2; }
+// Whether full RAVU r2 re-decides a wave's near sites together (wave_tensor), as r3 and r4 do,
+// or each lane its own: together where a sample is the FP64 luma of three (r2 rgb 2 x 1080p
+// 135.5 -> 117.5 us); otherwise its 16 points are soon done, and several of its lanes are near
+// at once (r2 luma together: 99.1 -> 131.9).
+template <int CH>
+constexpr bool wave_redecide() { return CH == 2; }
 
 // Hash of the site whose N x N window starts at staged-tile offset o (sample i at
 // o + (i % N) * PW + i / N), with the FP64 re-decision out of line: it is rare, and inlined
@@ -95,7 +92,7 @@ __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o)
 template <int N, int CH, int PW, int PN>
 __device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
   auto sample = [&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); };
-  if constexpr (wave_redecide<N, CH>()) {
+  if constexpr (wave_redecide<CH>()) {
     return ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
       const float* w = t + from_lane(o, site);
       return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
@@ -269,7 +266,7 @@ __device__ __forceinline__ void ravu_taps(const __half* lrow, S s, float* res) {
   for (int c = 0; c < P; ++c) res[c] = fminf(fmaxf(res[c], 0.f), 1.f);
 }
 
-// step1: int11 from the N = 2R window at offsets -(R-1)..R (ravu-r3.hook:22-146).
+// step1 for r2: int11 from the N = 2R window at offsets -(R-1)..R (ravu-r3.hook:22-146).
 template <int R, int CH, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(6))) void ravu_step1_kernel(Io io, const __half* __restrict__ lut, float* int11,
                                                          int64_t int11_frame, int total) {
@@ -330,7 +327,7 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
   };
   auto sample = [&](int i) { return luma_f<CH>(src(i), 0, PN); };
   Bucket bk;
-  if constexpr (wave_redecide<N, CH>()) {
+  if constexpr (wave_redecide<CH>()) {
     bk = ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
       const int o = from_lane(base, site);
       return [hk, o](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
@@ -360,7 +357,7 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
   }
 }
 
-// Steps 2 and 3 of a tile: both read the same staged input and int11 tiles (lattice
+// Steps 2 and 3 of a tile for r2: both read the same staged input and int11 tiles (lattice
 // offsets -R..R), so one kernel stages them once and runs the two steps one after the
 // other per site; a scheduling barrier between them keeps one step's registers live at a
 // time.
@@ -401,19 +398,364 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
   lattice_site<R, CH, 3, PW, PN>(io, lut, hk, i11, base, ft, x, y, valid, plane);
 }
 
+// ----------------------------------------------------------------------------- separable tensor
+//
+// The structure tensor's Gaussian is a product of its two axes, and the derivative along X
+// (Y) depends on a point's X (Y) index only through its stencil: central at the grid's first
+// and last index, five-point between (N = 6, 8).  So the sums over Y of one window column,
+//   A_t = sum_Y g(Y) gx_t^2,  B_t = sum_Y g(Y) c(Y) gx_t gy,  D = sum_Y g(Y) c(Y)^2 gy^2
+// for both stencils t of gx (unscaled derivatives, c = the stencil's scale) are shared by
+// the M = N - 2 windows that hold the column; a block tabulates them once in LDS and a site adds
+// M table entries per sum:
+//   a = sum_X g(X) c(X)^2 A_t(X),  b = sum_X g(X) c(X) B_t(X),  d = sum_X g(X) D.
+// Bound by VALU issue: the M^2 points evaluated per site took 358 instructions (r4), the table
+// and its sums take about 130 (with the shared tap columns: r4 4 x 1080p 292.6 -> 213.7 us, r4-yuv
+// 2 x 1080p 223.7 -> 195.9, r3 4 x 1080p 178.9 -> 163.7).  r2's window has border stencils at
+// every second point, so its columns would share too little: it keeps the sums per site.  The
+// order of the sums is free, as every decision within its error margin is re-made in FP64.
+template <int N>
+struct SepTensor {
+  static_assert(N == 6 || N == 8, "one inner and one outer stencil");
+  static constexpr int M = N - 2;  // grid positions 1 .. N - 2 of the window
+  __device__ static constexpr bool five(int i) { return i >= 1 && i + 3 <= M + 1; }  // grid index i = position i + 1
+  __device__ static constexpr double c(int i) { return five(i) ? 1.0 / 12.0 : 0.5; }
+  __device__ static constexpr double g(int i) {  // 1-D weight: the normalised grid's row sum
+    double s = 0;
+    for (int j = 0; j < M; ++j) s += gauss_w<N>(i * M + j);
+    return s;
+  }
+  // whether some of RUN successive columns sums uses stencil `f` of gy at row r of the run
+  template <int RUN>
+  __device__ static constexpr bool uses(bool f, int r) {
+    for (int k = 0; k < RUN; ++k)
+      if (r - k >= 0 && r - k < M && five(r - k) == f) return true;
+    return false;
+  }
+
+  struct Column {
+    float2 c, f;  // (A, B) for the central and the five-point gx
+    float d;
+  };
+  // Columns sums of RUN successive windows along Y: s(dx, dy) is the sample dx, dy steps from the
+  // first window's first grid row.
+  template <int RUN, typename S>
+  __device__ __forceinline__ static void columns(S s, Column (&out)[RUN]) {
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) out[k] = {{0.f, 0.f}, {0.f, 0.f}, 0.f};
+#pragma unroll
+    for (int r = 0; r < M + RUN - 1; ++r) {
+      const float xc = s(1, r) - s(-1, r);
+      const float xf = fmaf(8.0f, xc, s(-2, r) - s(2, r));
+      const float yc = s(0, r + 1) - s(0, r - 1);
+      float yf = 0.f;
+      if (uses<RUN>(true, r)) yf = fmaf(8.0f, yc, s(0, r - 2) - s(0, r + 2));
+      const float xc2 = xc * xc, xf2 = xf * xf;
+      const float cc = xc * yc, fc = xf * yc, yc2 = yc * yc;
+      const float cf = xc * yf, ff = xf * yf, yf2 = yf * yf;
+#pragma unroll
+      for (int k = 0; k < RUN; ++k) {
+        const int i = r - k;
+        if (i < 0 || i >= M) continue;
+        const float w = static_cast<float>(g(i)), wc = static_cast<float>(g(i) * c(i));
+        const float wcc = static_cast<float>(g(i) * c(i) * c(i));
+        out[k].c.x = fmaf(w, xc2, out[k].c.x);
+        out[k].f.x = fmaf(w, xf2, out[k].f.x);
+        out[k].c.y = fmaf(wc, five(i) ? cf : cc, out[k].c.y);
+        out[k].f.y = fmaf(wc, five(i) ? ff : fc, out[k].f.y);
+        out[k].d = fmaf(wcc, five(i) ? yf2 : yc2, out[k].d);
+      }
+    }
+  }
+  // a, b, d of one site: ab(five, X) returns the (A, B) entry of grid index X, dd(X) its D
+  template <typename AB, typename DD>
+  __device__ __forceinline__ static void site(AB ab, DD dd, float& a, float& b, float& d) {
+    a = b = d = 0.f;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const float2 e = ab(five(i), i);
+      a = fmaf(static_cast<float>(g(i) * c(i) * c(i)), e.x, a);
+      b = fmaf(static_cast<float>(g(i) * c(i)), e.y, b);
+      d = fmaf(static_cast<float>(g(i)), dd(i), d);
+    }
+  }
+};
+
+// Weight p (texel p / 4, component p % 4) of a LUT row held raw.
+template <int NTEX>
+struct RawRow {
+  uint2 t[NTEX];
+  __device__ __forceinline__ explicit RawRow(const __half* row) {
+    const uint2* r = reinterpret_cast<const uint2*>(row);
+#pragma unroll
+    for (int i = 0; i < NTEX; ++i) t[i] = r[i];
+  }
+  __device__ __forceinline__ float w(int p) const {
+    const __half2 h = bits_h2(p % 4 < 2 ? t[p / 4].x : t[p / 4].y);
+    return p % 2 ? __high2float(h) : __low2float(h);
+  }
+};
+
+__device__ __forceinline__ float clamp01(float v) { return fminf(fmaxf(v, 0.f), 1.f); }
+
+// step1 for r3 / r4, two vertically neighbouring sites per thread (TX x TY sites, TX * TY / 2
+// threads): the tap windows share N of their N + 1 rows, so a pair reads N (N + 1) samples
+// per plane from LDS instead of 2 N^2 (r4 yuv: LDS was busy 57 of 107 us).
+template <int R, int CH, int TX, int TY>
+__global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))) void ravu_step1_pair_kernel(
+    Io io, const __half* __restrict__ lut, float* int11, int64_t int11_frame, int total) {
+  constexpr int P = CH == 0 ? 1 : 3;
+  constexpr int N = 2 * R, NT = TX * TY / 2;
+  constexpr int PW = staged_width(TX + N - 1), PH = TY + N - 1, PN = PW * PH;
+  using Sep = SepTensor<N>;
+  constexpr int RUN = 4, NC = TX + Sep::M - 1;  // table columns: staged columns 1 .. NC
+  static_assert(TY % RUN == 0, "whole runs");
+  __shared__ __attribute__((aligned(16))) float tile[staged_planes<CH>() * PN];
+  __shared__ float2 tc[NC * TY], tf[NC * TY];
+  __shared__ float td[NC * TY];
+  const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
+  const int f = ft.f;
+  const int x0 = ft.x0, y0 = ft.y0;
+  stage_planes<P, PH, PW, NT>(tile, frame_in(io, f), io.in_dt, io.in_max, io.in_rmax, ft.in_pitch, ft.in_cstride,
+                              ft.W, ft.H, x0 - (R - 1), y0 - (R - 1));
+  __syncthreads();
+  if constexpr (CH == 2) {
+    stage_luma<CH>(tile, PN);
+    __syncthreads();
+  }
+  const float* lum = tile + (CH == 2 ? 3 * PN : 0);
+  for (int i = threadIdx.x; i < NC * (TY / RUN); i += NT) {
+    const int q = i / NC, c = i - q * NC;
+    const float* p = lum + (q * RUN + 1) * PW + c + 1;
+    typename Sep::Column v[RUN];
+    Sep::template columns<RUN>([&](int dx, int dy) { return p[dy * PW + dx]; }, v);
+#pragma unroll
+    for (int k = 0; k < RUN; ++k) {
+      const int e = (q * RUN + k) * NC + c;
+      tc[e] = v[k].c;
+      tf[e] = v[k].f;
+      td[e] = v[k].d;
+    }
+  }
+  __syncthreads();
+  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX * 2;
+  const int x = x0 + tx, y = y0 + ty;
+  const bool valid = x < ft.W && y < ft.H, second = y + 1 < ft.H;
+  const int o = ty * PW + tx;
+  int row[2] = {0, 0};
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int e = (ty + s) * NC + tx;
+    float a, b, d;
+    Sep::site([&](bool five, int i) { return five ? tf[e + i] : tc[e + i]; }, [&](int i) { return td[e + i]; }, a, b, d);
+    bool near = false;
+    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
+    redecide<N, true, RULE_LOG2>(near && valid && (s == 0 || second), [&](int site) {
+      const float* w = tile + from_lane(o, site) + s * PW;
+      return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
+    }, bk);
+    row[s] = bucket_row<RULE_LOG2>(bk, 648);
+    if (io.buckets && valid && (s == 0 || second))
+      io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y + s) * ft.W + x] = row[s];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (!valid) return;
+  constexpr int NTEX = RavuLut<N>::NTEX;
+  const RawRow<NTEX> w0(lut + row[0] * (NTEX * 4)), w1(lut + row[1] * (NTEX * 4));
+  const int64_t plane = static_cast<int64_t>(ft.W) * ft.H;
+  float* out = int11 + f * int11_frame + static_cast<int64_t>(y) * ft.W + x;
+  // res = sum over p < N^2/2 of (s_p + s_{N^2-1-p}) w_p, in order (ravu-r3.hook:120-146)
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    const float* p = tile + c * PN + o;
+    float r0 = 0.f, r1 = 0.f;
+#pragma unroll
+    for (int X = 0; X < N / 2; ++X) {
+      __builtin_amdgcn_sched_barrier(0);  // one column pair's samples live at a time
+      float l[N + 1], h[N + 1];
+#pragma unroll
+      for (int Y = 0; Y <= N; ++Y) {
+        l[Y] = p[Y * PW + X];
+        h[Y] = p[Y * PW + N - 1 - X];
+      }
+#pragma unroll
+      for (int Y = 0; Y < N; ++Y) {
+        r0 = fmaf(l[Y] + h[N - 1 - Y], w0.w(X * N + Y), r0);
+        r1 = fmaf(l[Y + 1] + h[N - Y], w1.w(X * N + Y), r1);
+      }
+      asm volatile("" : "+v"(r0), "+v"(r1));
+    }
+    r0 = clamp01(r0);
+    r1 = clamp01(r1);
+    out[c * plane] = io.store16 ? static_cast<float>(static_cast<_Float16>(r0)) : r0;
+    if (second) out[c * plane + ft.W] = io.store16 ? static_cast<float>(static_cast<_Float16>(r1)) : r1;
+  }
+}
+
+// Steps 2 and 3 for r3 / r4.  Lattice column L of pixel (x, y) holds the samples
+// (x + (L + Y - N + 2) / 2, y + (Y - L) / 2), Y = 0 .. N - 1; step 2's window is columns
+// 0 .. N - 1 and step 3's is columns -1 .. N - 2 (lat2x, lat2y), so the two share all but one.
+// The column sums of the tensor are tabulated by the column's first grid point (Y = 1): an
+// input pixel (i, j) for odd L, an int11 site (i + 1/2, j + 1/2) for even L, the next point
+// along Y; one thread sums the pair.
+template <int R, int CH, int TX, int TY>
+__global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const __half* __restrict__ lut,
+                                                                    const float* __restrict__ int11,
+                                                                    int64_t int11_frame, int total) {
+  constexpr int P = CH == 0 ? 1 : 3;
+  constexpr int N = 2 * R, NT = TX * TY;
+  constexpr int PW = staged_width(TX + 2 * R + 1), PH = TY + 2 * R + 1, PN = PW * PH;  // offsets -R..R
+  using Sep = SepTensor<N>;
+  constexpr int H = Sep::M / 2;
+  // tables by int11 site (-H .. TX - 1, -H .. TY - 1) and input pixel (1-H .. TX - 1, 1-H .. TY - 1)
+  constexpr int NC = TX + H, NR = TY + H, EC = NC - 1, ER = NR - 1, EN = EC * ER, TN = EN + NC * NR;
+  __shared__ __attribute__((aligned(16))) float tiles[2][staged_planes<CH>() * PN];
+  float *hk = tiles[0], *i11 = tiles[1];  // input (HOOKED), ravu_int11
+  __shared__ float2 tc[TN], tf[TN];  // input pixels' entries, then int11 sites'
+  __shared__ float td[TN];
+  const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
+  const int f = ft.f;
+  const int x0 = ft.x0, y0 = ft.y0;
+  const int64_t plane = static_cast<int64_t>(ft.W) * ft.H;
+  {
+    HaloTile<P, PH, PW, NT> a, b;  // both tiles' loads in flight together
+    __builtin_amdgcn_s_setprio(1);  // the loads go out ahead of other waves' arithmetic
+    a.issue(frame_in(io, f), io.in_dt, ft.in_pitch, ft.in_cstride, ft.W, ft.H, x0 - R, y0 - R);
+    b.issue(int11 + f * int11_frame, DT_F32, ft.W, plane, ft.W, ft.H, x0 - R, y0 - R);
+    __builtin_amdgcn_s_setprio(0);
+    a.commit(hk, io.in_dt, io.in_max, io.in_rmax, ft.W, x0 - R);
+    b.commit(i11, DT_F32, 1.f, 1.f, ft.W, x0 - R);
+  }
+  __syncthreads();
+  if constexpr (CH == 2) {
+    stage_luma<CH>(hk, PN);
+    stage_luma<CH>(i11, PN);
+    __syncthreads();
+  }
+  {
+    const float* lh = hk + (CH == 2 ? 3 * PN : 0);
+    const float* li = i11 + (CH == 2 ? 3 * PN : 0);
+    for (int i = threadIdx.x; i < NC * NR; i += NT) {
+      const int q = i / NC, c = i - q * NC;
+      const int o = (q - H + R) * PW + c - H + R;  // input pixel (c - H, q - H)
+      typename Sep::Column v[2];
+      Sep::template columns<2>(
+          [&](int dx, int dy) {  // lattice steps from that pixel
+            const int u = dx + dy, w = dy - dx;
+            return (u & 1) ? li[o + ((w - 1) >> 1) * PW + ((u - 1) >> 1)] : lh[o + (w >> 1) * PW + (u >> 1)];
+          },
+          v);
+      if (q > 0 && c > 0) {
+        const int e = (q - 1) * EC + c - 1;
+        tc[e] = v[0].c;
+        tf[e] = v[0].f;
+        td[e] = v[0].d;
+      }
+      tc[EN + i] = v[1].c;
+      tf[EN + i] = v[1].f;
+      td[EN + i] = v[1].d;
+    }
+  }
+  __syncthreads();
+  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+  const int x = x0 + tx, y = y0 + ty;
+  const bool valid = x < ft.W && y < ft.H;
+  const int base = (ty + R) * PW + tx + R;  // LDS offset of (x, y)
+  const int ee = (ty + H - 1) * EC + tx + H - 1, oe = EN + (ty + H) * NC + tx + H;  // table entries of (x, y)
+  // table entry of column L (0 .. M): input pixel (x + (L - N + 3) / 2, y + (1 - L) / 2) for odd
+  // L, int11 site (x + (L - N + 2) / 2, y - L / 2) for even L
+  auto entry = [&](int L) {
+    return L & 1 ? ee + (L - N + 3) / 2 + (1 - L) / 2 * EC : oe + (L - N + 2) / 2 - L / 2 * NC;
+  };
+  auto src = [&](int L, int Y) -> const float* {
+    const int px = L + Y - N + 2, py = Y - L;
+    return (px & 1) ? i11 + base + ((py - 1) >> 1) * PW + ((px - 1) >> 1) : hk + base + (py >> 1) * PW + (px >> 1);
+  };
+  int row[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {  // step 2, step 3: grid index i is column i + 1, i
+    float a, b, d;
+    Sep::site([&](bool five, int i) {
+          return five ? tf[entry(i + 1 - s)] : tc[entry(i + 1 - s)];
+        },
+        [&](int i) { return td[entry(i + 1 - s)]; }, a, b, d);
+    bool near = false;
+    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
+    redecide<N, true, RULE_LOG2>(near && valid, [&](int site) {
+      const int o = from_lane(base, site);
+      return [hk, o, s](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
+        const int px = X - s + Y - N + 2, py = Y - X + s;
+        return luma_d<CH>(hk, o + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
+      };
+    }, bk);
+    row[s] = bucket_row<RULE_LOG2>(bk, 648);
+    if (io.buckets && valid)
+      io.buckets[f * io.bucket_bstride + (s + 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row[s];
+    __builtin_amdgcn_sched_barrier(0);  // one step's registers live at a time
+  }
+  if (!valid) return;
+  constexpr int NTEX = RavuLut<N>::NTEX;
+  const RawRow<NTEX> w2(lut + row[0] * (NTEX * 4)), w3(lut + row[1] * (NTEX * 4));
+  const int esz_out = elem_bytes(io.out_dt);
+  char* ob = static_cast<char*>(frame_out(io, f));
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    // step 2 pairs columns (X, N-1-X), step 3 (X-1, N-2-X): each column is read once for both
+    float r2 = 0.f, r3 = 0.f, below[N], high[N];
+#pragma unroll
+    for (int Y = 0; Y < N; ++Y) {
+      below[Y] = src(-1, Y)[c * PN];
+      high[Y] = src(N - 1, Y)[c * PN];
+    }
+#pragma unroll
+    for (int X = 0; X < N / 2; ++X) {
+      __builtin_amdgcn_sched_barrier(0);
+      float low[N], next[N];
+#pragma unroll
+      for (int Y = 0; Y < N; ++Y) {
+        low[Y] = src(X, Y)[c * PN];
+        next[Y] = X + 1 < N / 2 ? src(N - 2 - X, Y)[c * PN] : low[Y];
+      }
+#pragma unroll
+      for (int Y = 0; Y < N; ++Y) {
+        r2 = fmaf(low[Y] + high[N - 1 - Y], w2.w(X * N + Y), r2);
+        r3 = fmaf(below[Y] + next[N - 1 - Y], w3.w(X * N + Y), r3);
+      }
+      asm volatile("" : "+v"(r2), "+v"(r3));
+#pragma unroll
+      for (int Y = 0; Y < N; ++Y) {
+        below[Y] = low[Y];
+        high[Y] = next[Y];
+      }
+    }
+    void* o = ob + c * ft.out_cstride * esz_out;
+    const int64_t at = static_cast<int64_t>(2 * y) * ft.out_pitch + 2 * x;
+    // the combine pass (ravu-r3.hook:426-437): rows (input, int10) and (int01, int11)
+    store_pair(o, at, io.out_dt, hk[c * PN + base], clamp01(r2));
+    store_pair(o, at + ft.out_pitch, io.out_dt, clamp01(r3), i11[c * PN + base]);
+  }
+}
+
 template <int T>
 static hipError_t launch_ravu_tile(int r, int channels, Io io, const __half* lut, float* int11, int64_t int11_frame,
                                    hipStream_t st, hipEvent_t done) {
   constexpr int TX = kRavuTiles[T].w, TY = kRavuTiles[T].h;
   const int total = launch_tiles<TX, TY>(io);
   const dim3 grid(total), block(TX * TY);
-#define MPX_RAVU(R, CH)                                                                                         \
-  if (r == R && channels == CH) {                                                                               \
-    hipLaunchKernelGGL((ravu_step1_kernel<R, CH, TX, TY>), grid, block, 0, st, io, lut, int11, int11_frame, total); \
-    hipError_t e = hipGetLastError();                                                                           \
-    if (e != hipSuccess) return e;                                                                              \
-    return launch_done(ravu_lattice_kernel<R, CH, TX, TY>, grid, block, st, done, io, lut, int11, int11_frame,      \
-                       total);                                                                                  \
+#define MPX_RAVU(R, CH)                                                                                            \
+  if (r == R && channels == CH) {                                                                                  \
+    if constexpr (R >= 3)                                                                                          \
+      hipLaunchKernelGGL((ravu_step1_pair_kernel<R, CH, TX, TY>), grid, dim3(TX * TY / 2), 0, st, io, lut, int11,   \
+                         int11_frame, total);                                                                      \
+    else                                                                                                           \
+      hipLaunchKernelGGL((ravu_step1_kernel<R, CH, TX, TY>), grid, block, 0, st, io, lut, int11, int11_frame, total); \
+    hipError_t e = hipGetLastError();                                                                              \
+    if (e != hipSuccess) return e;                                                                                 \
+    if constexpr (R >= 3)                                                                                          \
+      return launch_done(ravu_lattice_pair_kernel<R, CH, TX, TY>, grid, block, st, done, io, lut, int11,            \
+                         int11_frame, total);                                                                      \
+    else                                                                                                           \
+      return launch_done(ravu_lattice_kernel<R, CH, TX, TY>, grid, block, st, done, io, lut, int11, int11_frame,    \
+                         total);                                                                                   \
   }
   MPX_RAVU(2, 0) MPX_RAVU(2, 1) MPX_RAVU(2, 2) MPX_RAVU(3, 0) MPX_RAVU(3, 1) MPX_RAVU(3, 2) MPX_RAVU(4, 0)
   MPX_RAVU(4, 1) MPX_RAVU(4, 2)
@@ -424,7 +766,7 @@ static hipError_t launch_ravu_tile(int r, int channels, Io io, const __half* lut
 hipError_t launch_ravu(int r, int channels, const Io& io, const __half* lut, float* int11, int64_t int11_frame,
                        int tile, hipStream_t st, hipEvent_t done) {
   static_assert(kRavuTileCount == 3, "one case per tile shape");
-  switch (tile) {
+  switch (ravu_tile_index(r, channels, tile)) {
     case 0: return launch_ravu_tile<0>(r, channels, io, lut, int11, int11_frame, st, done);
     case 1: return launch_ravu_tile<1>(r, channels, io, lut, int11, int11_frame, st, done);
     case 2: return launch_ravu_tile<2>(r, channels, io, lut, int11, int11_frame, st, done);
