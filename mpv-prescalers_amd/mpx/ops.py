@@ -16,6 +16,20 @@ from ._abi import LIB, MpxError, MpxIo, VariantInfo, check
 
 _DT = {torch.uint8: _abi.U8, torch.uint16: _abi.U16, torch.float16: _abi.F16, torch.float32: _abi.F32}
 
+# The current stream's handle and the current device straight from the runtime: the Stream
+# object that torch.cuda.current_stream builds takes 1.9 us, a call of a small frame about 10.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def _stream_handle(x, stream):
+    """hipStream_t (as an int) of ``stream``, or of the current stream of ``x``'s device."""
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is not None:
+        return _raw_stream(x.get_device())
+    return torch.cuda.current_stream(x.device).cuda_stream
+
 
 def variants():
     """All shipped variant names (46), including the three ravu-zoom-ar-r3 forms whose
@@ -82,9 +96,7 @@ class Plan:
         """Upscale ``x`` (device tensor) into ``out`` (allocated if None).  Returns ``out``,
         or ``(out, bucket_rows)`` with ``buckets=True``."""
         io, x, out, bk = self._io(x, out, buckets)
-        if stream is None:
-            stream = torch.cuda.current_stream(x.device)
-        check(LIB.mpx_run_ex(self._h, ctypes.byref(io), ctypes.c_void_p(stream.cuda_stream)))
+        check(LIB.mpx_run_ex(self._h, io, _stream_handle(x, stream)))
         return (out, bk) if buckets else out
 
     def run_static(self, x, out=None, stream=None):
@@ -93,9 +105,7 @@ class Plan:
         call allocates nothing but ``out`` when it is None.  Calls that overlap on one
         device race on that array."""
         io, x, out, _ = self._io(x, out, False)
-        if stream is None:
-            stream = torch.cuda.current_stream(x.device)
-        check(LIB.mpx_run_static(self._h, ctypes.byref(io), ctypes.c_void_p(stream.cuda_stream)))
+        check(LIB.mpx_run_static(self._h, io, _stream_handle(x, stream)))
         return out
 
     def tune(self, x, out=None, iters=5, stream=None):
@@ -149,41 +159,40 @@ class Plan:
         planes = self.info["planes"]
         if x.dtype != self.in_dtype:
             raise TypeError("plan expects %s input, got %s" % (self.in_dtype, x.dtype))
-        if x.shape[-2:] != (self.in_h, self.in_w):
-            raise ValueError("plan expects %dx%d input, got %s" % (self.in_w, self.in_h, tuple(x.shape)))
+        shape = x.shape
+        if shape[-2:] != (self.in_h, self.in_w):
+            raise ValueError("plan expects %dx%d input, got %s" % (self.in_w, self.in_h, tuple(shape)))
         if not x.is_cuda:
             raise ValueError("input must be a device tensor")
         nd = 2 if planes == 1 else 3
-        if x.dim() == nd:
+        dim = len(shape)
+        if dim == nd:
             batch = 1
-        elif x.dim() == nd + 1:
-            batch = x.shape[0]
+        elif dim == nd + 1:
+            batch = shape[0]
         else:
-            raise ValueError("bad input rank %d" % x.dim())
-        if planes == 3 and x.shape[-3] != 3:
+            raise ValueError("bad input rank %d" % dim)
+        if planes == 3 and shape[-3] != 3:
             raise ValueError("3-plane variant expects 3 planes")
-        if x.stride(-1) != 1:
+        ist = x.stride()
+        if ist[-1] != 1:
             x = x.contiguous()
+            ist = x.stride()
+        oh, ow = self.info["out_h"], self.info["out_w"]
         if out is None:
-            out = torch.empty(self.out_shape(x), dtype=self.out_dtype, device=x.device)
-        if out.stride(-1) != 1 or out.dtype != self.out_dtype or tuple(out.shape) != self.out_shape(x):
-            raise ValueError("bad output tensor")
+            out = torch.empty(shape[:-2] + (oh, ow), dtype=self.out_dtype, device=x.device)
+            ost = out.stride()
+        else:
+            ost = out.stride()
+            if ost[-1] != 1 or out.dtype != self.out_dtype or tuple(out.shape) != self.out_shape(x):
+                raise ValueError("bad output tensor")
         bk = None
         if buckets:
             bk = torch.empty((batch, self.bucket_count), dtype=torch.int32, device=x.device)
-        io = MpxIo()
-        io.in_ = x.data_ptr()
-        io.in_pitch = x.stride(-2)
-        io.in_cstride = x.stride(-3) if planes == 3 else x.stride(-2) * self.in_h
-        io.in_bstride = x.stride(0) if x.dim() == nd + 1 else x.numel()
-        io.out = out.data_ptr()
-        io.out_pitch = out.stride(-2)
-        io.out_cstride = out.stride(-3) if planes == 3 else out.stride(-2) * self.info["out_h"]
-        io.out_bstride = out.stride(0) if out.dim() == nd + 1 else out.numel()
-        io.batch = batch
-        io.buckets = bk.data_ptr() if bk is not None else None
-        return io, x, out, bk
-
+        return MpxIo(x.data_ptr(), ist[-2], ist[-3] if planes == 3 else ist[-2] * self.in_h,
+                     ist[0] if dim > nd else x.numel(), out.data_ptr(), ost[-2],
+                     ost[-3] if planes == 3 else ost[-2] * oh, ost[0] if dim > nd else out.numel(), batch,
+                     bk.data_ptr() if bk is not None else None), x, out, bk
 
     def run_frames(self, xs, outs=None, stream=None):
         """One launch (per pass) over separate same-shape frames (up to 16): each x in
@@ -210,9 +219,7 @@ class Plan:
                 raise ValueError("frames must share row pitches")
         ins = (ctypes.c_void_p * n)(*[x.data_ptr() for x in xs])
         ots = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-        if stream is None:
-            stream = torch.cuda.current_stream(xs[0].device)
-        check(LIB.mpx_run_frames(self._h, n, ins, ots, pitch_in, pitch_out, ctypes.c_void_p(stream.cuda_stream)))
+        check(LIB.mpx_run_frames(self._h, n, ins, ots, pitch_in, pitch_out, _stream_handle(xs[0], stream)))
         return outs
 
 
@@ -245,9 +252,7 @@ class Plan:
         hs = (ctypes.c_int * n)(*[x.shape[-2] for x in xs])
         ips = (ctypes.c_int64 * n)(*[x.stride(-2) for x in xs])
         ops_ = (ctypes.c_int64 * n)(*[o.stride(-2) for o in outs])
-        if stream is None:
-            stream = torch.cuda.current_stream(xs[0].device)
-        check(LIB.mpx_run_frames_sized(self._h, n, ins, ots, ws, hs, ips, ops_, ctypes.c_void_p(stream.cuda_stream)))
+        check(LIB.mpx_run_frames_sized(self._h, n, ins, ots, ws, hs, ips, ops_, _stream_handle(xs[0], stream)))
         return outs
 
 
@@ -366,10 +371,11 @@ def _resample(x, size, offset, filter, out_dtype, bits, stream, planes):
     io.out_cstride = out.stride(-3) if planes == 3 else out.stride(-2) * out_h
     io.out_bstride = out.stride(0) if x.dim() == nd + 1 else out.numel()
     io.batch = batch
-    if stream is None:
-        stream = torch.cuda.current_stream(x.device)
-    with torch.cuda.device(x.device):
-        check(LIB.mpx_resample(ctypes.byref(io), in_w, in_h, _DT[x.dtype], bits, out_w, out_h, _DT[out_dtype], planes,
-                               _abi.FILTER[filter], float(offset[0]), float(offset[1]),
-                               ctypes.c_void_p(stream.cuda_stream)))
+    args = (io, in_w, in_h, _DT[x.dtype], bits, out_w, out_h, _DT[out_dtype], planes, _abi.FILTER[filter],
+            float(offset[0]), float(offset[1]), _stream_handle(x, stream))
+    if _raw_device is not None and _raw_device() == x.get_device():
+        check(LIB.mpx_resample(*args))
+    else:
+        with torch.cuda.device(x.device):
+            check(LIB.mpx_resample(*args))
     return out
