@@ -361,28 +361,22 @@ __device__ __forceinline__ T div_const(T x, T b, T rb) {
 
 // Derivative along one window line at position p, in the shaders' formula forms
 // (ravu-lite-r3.hook:50 central; ravu-r3.hook:64 five-point; ravu-zoom-r2.hook:50
-// forward/backward at the window border).  `s(k)` returns the line's k-th sample.
-template <int N, bool FIVE, typename T, typename Line>
-__device__ __forceinline__ T deriv(Line s, int p) {
+// forward/backward at the window border), in FP64 (the re-decision): the correctly rounded
+// quotients, as the oracle's divisions give.  `s(k)` returns the line's k-th sample.
+template <int N, bool FIVE, typename Line>
+__device__ __forceinline__ double deriv(Line s, int p) {
 #pragma clang fp contract(off)
   if (p == 0) return s(1) - s(0);
   if (p == N - 1) return s(N - 1) - s(N - 2);
-  // FP32 (the fast path, whose decisions are trusted only away from bucket boundaries)
-  // multiplies by the reciprocals: exact for 1/2, within one rounding of the quotient for
-  // 1/12.  FP64 (the re-decision) gives the correctly rounded quotient, as the oracle's
-  // division does.
   if (FIVE && p >= 2 && p + 2 <= N - 1) {
-    if constexpr (sizeof(T) == 4)  // same value, fused: (s[p-2] - s[p+2]) + 8 (s[p+1] - s[p-1])
-      return fmaf(8.0f, s(p + 1) - s(p - 1), s(p - 2) - s(p + 2)) * (1.0f / 12.0f);
-    const T num = -s(p + 2) + T(8) * s(p + 1) - T(8) * s(p - 1) + s(p - 2);
-    return div_const(num, T(12), T(1) / T(12));
+    const double num = -s(p + 2) + 8.0 * s(p + 1) - 8.0 * s(p - 1) + s(p - 2);
+    return div_const(num, 12.0, 1.0 / 12.0);
   }
-  if constexpr (sizeof(T) == 4) return (s(p + 1) - s(p - 1)) * T(0.5);
-  return (s(p + 1) - s(p - 1)) / T(2);
+  return (s(p + 1) - s(p - 1)) / 2.0;
 }
 
-// The same derivatives without their stencil's scale (FP32 fast path), and that scale:
-// 1 at the window border (forward/backward), 1/12 for the five-point form, 1/2 central.
+// The derivatives of the FP32 fast path without their stencil's scale, and that scale: 1 at
+// the window border (forward/backward), 1/12 for the five-point form, 1/2 central.
 template <int N, bool FIVE>
 __device__ __host__ constexpr double deriv_scale(int p) {
   return (p == 0 || p == N - 1) ? 1.0 : (FIVE && p >= 2 && p + 2 <= N - 1) ? 1.0 / 12.0 : 0.5;
@@ -395,62 +389,6 @@ __device__ __forceinline__ float deriv_unscaled(Line s, int p) {
   return s(p + 1) - s(p - 1);
 }
 
-// abd = sum over the gradient grid of (gx*gx, gx*gy, gy*gy) * G, grid X outer, Y inner
-// (ravu-lite-r3.hook:48-76).  get(i) returns window sample i = X*N + Y.  FP32 (the fast
-// path, trusted only away from bucket boundaries) fuses multiply-adds; FP64 (the
-// re-decision) keeps every rounding step of the formula, like the oracle.
-// LEAN (the full-RAVU kernels, whose windows are largest) trims both: FP32 takes the
-// derivatives unscaled and folds each point's stencil scales into its Gaussian weight
-// (compile-time constants), and where gx and gy carry the same scale one product w'*gx
-// serves both a and b; FP64 is computed one derivative at a time (scheduling barriers,
-// the partial sums pinned), so the rare re-decision does not hold the window in FP64
-// registers and set the occupancy of every wave (r4: 122 -> 58 VGPRs).  The sums keep
-// the oracle's order either way.
-template <int N, bool FIVE, typename T, bool LEAN, typename Get>
-__device__ __forceinline__ void structure_tensor(Get get, T& a, T& b, T& d) {
-#pragma clang fp contract(off)
-  constexpr int P0 = N <= 4 ? 0 : 1;
-  constexpr int P1 = N <= 4 ? N : N - 1;
-  a = b = d = T(0);
-#pragma unroll
-  for (int X = P0; X < P1; ++X) {
-#pragma unroll
-    for (int Y = P0; Y < P1; ++Y) {
-      const int gi = (X - P0) * (P1 - P0) + (Y - P0);
-      if constexpr (sizeof(T) == 4 && LEAN) {
-        const float gx = deriv_unscaled<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
-        const float gy = deriv_unscaled<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
-        const double cx = deriv_scale<N, FIVE>(X), cy = deriv_scale<N, FIVE>(Y), w = gauss_w<N>(gi);
-        const float u = gx * static_cast<float>(w * cx * cx);
-        a = fmaf(u, gx, a);
-        b = cx == cy ? fmaf(u, gy, b) : fmaf(gx * static_cast<float>(w * cx * cy), gy, b);
-        d = fmaf(gy * static_cast<float>(w * cy * cy), gy, d);
-        continue;
-      }
-      T gx = deriv<N, FIVE, T>([&](int k) { return get(k * N + Y); }, X);
-      if constexpr (sizeof(T) == 8 && LEAN) {
-        asm volatile("" : "+v"(gx));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      T gy = deriv<N, FIVE, T>([&](int k) { return get(X * N + k); }, Y);
-      const T w = T(gauss_w<N>(gi));
-      if constexpr (sizeof(T) == 4) {  // fast path: fused accumulation
-        a = fmaf(gx * gx, w, a);
-        b = fmaf(gx * gy, w, b);
-        d = fmaf(gy * gy, w, d);
-      } else {                         // re-decision: the reference's rounding steps
-        a = a + gx * gx * w;
-        b = b + gx * gy * w;
-        d = d + gy * gy * w;
-        if constexpr (LEAN) {
-          asm volatile("" : "+v"(a), "+v"(b), "+v"(d));
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-    }
-  }
-}
-
 // Gradient grid of an N x N window: positions P0 .. P1 - 1 on both axes.
 template <int N>
 struct GradGrid {
@@ -458,6 +396,63 @@ struct GradGrid {
   static constexpr int P1 = N <= 4 ? N : N - 1;
   static constexpr int M = P1 - P0;
 };
+
+// abd = sum over the gradient grid of (gx*gx, gx*gy, gy*gy) * G, grid X outer, Y inner
+// (ravu-lite-r3.hook:48-76), FP32 fast path, trusted only away from bucket boundaries.  get(i)
+// returns window sample i = X*N + Y.  The derivatives are taken unscaled and each point's
+// stencil scales folded into its Gaussian weight (compile-time constants); where gx and gy
+// carry the same scale one product w'*gx serves both a and b (lite-r3 8 x 1080p 132.4 ->
+// 128.4 us, zoom-r2 4 x 720p -> 1440p 117.1 -> 113.3).
+template <int N, bool FIVE, typename Get>
+__device__ __forceinline__ void structure_tensor(Get get, float& a, float& b, float& d) {
+#pragma clang fp contract(off)
+  using GG = GradGrid<N>;
+  a = b = d = 0.f;
+#pragma unroll
+  for (int X = GG::P0; X < GG::P1; ++X) {
+#pragma unroll
+    for (int Y = GG::P0; Y < GG::P1; ++Y) {
+      const float gx = deriv_unscaled<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
+      const float gy = deriv_unscaled<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
+      const double cx = deriv_scale<N, FIVE>(X), cy = deriv_scale<N, FIVE>(Y);
+      const double w = gauss_w<N>((X - GG::P0) * GG::M + (Y - GG::P0));
+      const float u = gx * static_cast<float>(w * cx * cx);
+      a = fmaf(u, gx, a);
+      b = cx == cy ? fmaf(u, gy, b) : fmaf(gx * static_cast<float>(w * cx * cy), gy, b);
+      d = fmaf(gy * static_cast<float>(w * cy * cy), gy, d);
+    }
+  }
+}
+
+// The same in FP64, in the reference's rounding steps and order, by one lane.  LEAN (large
+// windows): one derivative at a time (scheduling barriers, the partial sums pinned), so the
+// rare re-decision does not hold the window in FP64 registers and set every wave's occupancy.
+template <int N, bool FIVE, bool LEAN, typename Get>
+__device__ __forceinline__ void structure_tensor_fp64(Get get, double& a, double& b, double& d) {
+#pragma clang fp contract(off)
+  using GG = GradGrid<N>;
+  a = b = d = 0.0;
+#pragma unroll
+  for (int X = GG::P0; X < GG::P1; ++X) {
+#pragma unroll
+    for (int Y = GG::P0; Y < GG::P1; ++Y) {
+      double gx = deriv<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
+      if constexpr (LEAN) {
+        asm volatile("" : "+v"(gx));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const double gy = deriv<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
+      const double w = gauss_w<N>((X - GG::P0) * GG::M + (Y - GG::P0));
+      a = a + gx * gx * w;
+      b = b + gx * gy * w;
+      d = d + gy * gy * w;
+      if constexpr (LEAN) {
+        asm volatile("" : "+v"(a), "+v"(b), "+v"(d));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+}
 
 enum Rule : int { RULE_LITE = 0, RULE_3X = 1, RULE_LOG2 = 2 };
 
@@ -688,12 +683,12 @@ __device__ __forceinline__ int from_lane(int v, int i) { return __builtin_amdgcn
 template <int N, bool FIVE, int RULE, bool LEAN = false, typename GetF, typename GetD>
 __device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
   float a, b, d;
-  structure_tensor<N, FIVE, float, LEAN>(getf, a, b, d);
+  structure_tensor<N, FIVE>(getf, a, b, d);
   bool near = false;
   Bucket bk = hash_fast<RULE>(a, b, d, &near);
   if (near) {
     double ad, bd, dd;
-    structure_tensor<N, FIVE, double, LEAN>(getd, ad, bd, dd);
+    structure_tensor_fp64<N, FIVE, LEAN>(getd, ad, bd, dd);
     bk = hash_reference<RULE, double>(ad, bd, dd);
   }
   return bk;
@@ -703,10 +698,10 @@ __device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
 // window sample i; at(site): see wave_tensor.  All lanes of the wave call it together; lanes
 // without a site (`valid` false) read their window too (inside the staged tile) but are never
 // re-decided.
-template <int N, bool FIVE, int RULE, bool LEAN, typename GetF, typename At>
+template <int N, bool FIVE, int RULE, typename GetF, typename At>
 __device__ __forceinline__ Bucket ravu_hash_wave(bool valid, GetF getf, At at) {
   float a, b, d;
-  structure_tensor<N, FIVE, float, LEAN>(getf, a, b, d);
+  structure_tensor<N, FIVE>(getf, a, b, d);
   bool near = false;
   Bucket bk = hash_fast<RULE>(a, b, d, &near);
   redecide<N, FIVE, RULE>(near && valid, at, bk);

@@ -47,7 +47,7 @@ inline hipError_t launch_done(K kern, dim3 grid, dim3 block, hipStream_t st, hip
 struct TileShape {
   int w, h;
 };
-constexpr TileShape kLiteTiles[] = {{64, 4}, {32, 8}, {32, 4}};
+constexpr TileShape kLiteTiles[] = {{32, 8}, {64, 4}, {32, 4}};
 constexpr TileShape k3xTiles[] = {{32, 8}, {64, 4}};
 constexpr TileShape kRavuTiles[] = {{32, 8}, {32, 16}, {64, 8}};
 constexpr TileShape kZoomTiles[] = {{32, 8}, {16, 16}};

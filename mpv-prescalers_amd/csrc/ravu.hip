@@ -84,7 +84,7 @@ constexpr bool wave_redecide() { return CH == 2; }
 template <int N, bool FIVE, int RULE, int CH, int PW, int PN>
 __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o) {
   double a, b, d;
-  structure_tensor<N, FIVE, double, true>([&](int s) { return luma_d<CH>(t, o + (s % N) * PW + s / N, PN); }, a, b,
+  structure_tensor_fp64<N, FIVE, true>([&](int s) { return luma_d<CH>(t, o + (s % N) * PW + s / N, PN); }, a, b,
                                           d);
   return hash_reference<RULE, double>(a, b, d);
 }
@@ -93,13 +93,13 @@ template <int N, int CH, int PW, int PN>
 __device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
   auto sample = [&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); };
   if constexpr (wave_redecide<CH>()) {
-    return ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
+    return ravu_hash_wave<N, true, RULE_LOG2>(valid, sample, [&](int site) {
       const float* w = t + from_lane(o, site);
       return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
     });
   } else {
     float a, b, d;
-    structure_tensor<N, true, float, true>(sample, a, b, d);
+    structure_tensor<N, true>(sample, a, b, d);
     bool near = false;
     const Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
     return near && valid ? redecide_site<N, true, RULE_LOG2, CH, PW, PN>(t, o) : bk;
@@ -141,19 +141,24 @@ __global__ __launch_bounds__(TX * TY) void ravu_3x_kernel(Io io, const __half* _
   for (int c = 0; c < P; ++c)
 #pragma unroll
     for (int k = 0; k < 4; ++k) r0[c][k] = r1[c][k] = 0.f;
-  // One step per tap pair (two LUT texels), software-pipelined: the next step's texels
-  // are fetched (as raw FP16, converted inside the multiply-adds) while this step
-  // computes, and each step's sums complete before the next step's samples are read, so
-  // only one step's operands are live (r3 luma: 46 VGPRs instead of 134).
+  // One step per tap pair (two LUT texels), software-pipelined: texels are fetched (as raw
+  // FP16, converted inside the multiply-adds) three steps ahead, and each step's sums
+  // complete before the next step's samples are read, so only one step's operands are live.
   const uint2* lraw = reinterpret_cast<const uint2*>(lrow);
-  uint2 t0 = lraw[0], t1 = lraw[1];
+  constexpr int AHEAD = 3;
+  uint2 q0[AHEAD], q1[AHEAD];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) {
+    q0[i] = lraw[2 * min(i, C)];
+    q1[i] = lraw[2 * min(i, C) + 1];
+  }
 #pragma unroll
   for (int i = 0; i <= C; ++i) {
     __builtin_amdgcn_sched_barrier(0);
-    uint2 n0 = t0, n1 = t1;
-    if (i < C) {
-      n0 = lraw[2 * i + 2];
-      n1 = lraw[2 * i + 3];
+    const uint2 t0 = q0[i % AHEAD], t1 = q1[i % AHEAD];
+    if (i + AHEAD <= C) {
+      q0[i % AHEAD] = lraw[2 * (i + AHEAD)];
+      q1[i % AHEAD] = lraw[2 * (i + AHEAD) + 1];
     }
     const __half2 h00 = bits_h2(t0.x), h01 = bits_h2(t0.y), h10 = bits_h2(t1.x), h11 = bits_h2(t1.y);
     const float a0[4] = {__low2float(h00), __high2float(h00), __low2float(h01), __high2float(h01)};
@@ -182,8 +187,6 @@ __global__ __launch_bounds__(TX * TY) void ravu_3x_kernel(Io io, const __half* _
     for (int c = 0; c < P; ++c)
 #pragma unroll
       for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(r0[c][k]), "+v"(r1[c][k]));
-    t0 = n0;
-    t1 = n1;
   }
   const int esz_out = elem_bytes(io.out_dt);
   char* ob = static_cast<char*>(frame_out(io, f));
@@ -328,7 +331,7 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
   auto sample = [&](int i) { return luma_f<CH>(src(i), 0, PN); };
   Bucket bk;
   if constexpr (wave_redecide<CH>()) {
-    bk = ravu_hash_wave<N, true, RULE_LOG2, true>(valid, sample, [&](int site) {
+    bk = ravu_hash_wave<N, true, RULE_LOG2>(valid, sample, [&](int site) {
       const int o = from_lane(base, site);
       return [hk, o](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
         const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);

@@ -122,7 +122,7 @@ __device__ __forceinline__ double zluma_d(const float* t, int o, int n) {
 template <int N, int CH, int PW, int PN, bool TAB>
 __device__ __attribute__((noinline)) int zoom_redecide(const float* t, int o) {
   double a, b, d;
-  structure_tensor<N, true, double, true>([&](int s) { return zluma_d<CH>(t, o + (s % N) * PW + s / N, PN); },
+  structure_tensor_fp64<N, true, true>([&](int s) { return zluma_d<CH>(t, o + (s % N) * PW + s / N, PN); },
                                           a, b, d);
   const Bucket bk = hash_reference<RULE_LITE, double>(a, b, d);
   return (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
@@ -288,14 +288,14 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
     int value;
     if constexpr (R >= 3 || AR || CH == 2) {
       const int origin = by * PW + bx;
-      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, (R >= 3)>(lane_i == i, sample, [&](int site) {
+      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE>(lane_i == i, sample, [&](int site) {
         const float* t = tile + from_lane(origin, site);
         return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
       });
       value = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
     } else {
       float ta, tb, td;
-      structure_tensor<N, true, float, false>(sample, ta, tb, td);
+      structure_tensor<N, true>(sample, ta, tb, td);
       bool near = false;
       const Bucket bk = hash_fast<RULE_LITE>(ta, tb, td, &near);
       value = near && lane_i == i ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
