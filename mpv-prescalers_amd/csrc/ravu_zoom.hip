@@ -241,6 +241,44 @@ __global__ __launch_bounds__(256) void zoom_phase_kernel(int4* tab, int in_w, in
   tab[i] = make_int4(ph.base, __float_as_int(ph.f), o % (x ? nphx : nphy), 0);
 }
 
+// Anti-ringing of one output: mix(res, clamp(res, lo, hi), 0.8), no final clamp.
+__device__ __forceinline__ float zoom_ring(float v, float hi, float lo, float hi2, float lo2) {
+  const float h = hi2 * __builtin_amdgcn_rcpf(hi) - 0.1f, l = 1.1f - lo2 * __builtin_amdgcn_rcpf(lo);
+  const float cl = fminf(fmaxf(v, l), h);
+  return v * (1.0f - 0.8f) + cl * 0.8f;
+}
+
+// Hash every base pixel of a tile (nbx x nby) into bucket[by * BX + bx]: the unclamped LUT row
+// (bucket 9-row blocks are clamped per texel by the bilinear fetch, as the sampler does).
+template <int R, bool AR, int CH, bool TAB, int BX, int PW, int PN, int NT>
+__device__ __forceinline__ void hash_bases(const float* tile, int* bucket, int nbx, int nby) {
+  constexpr int N = 2 * R;
+  // (whole waves: the re-decision takes all lanes; those past the last base pixel repeat it)
+  for (int i0 = threadIdx.x & ~63; i0 < nbx * nby; i0 += NT) {
+    const int lane_i = i0 + static_cast<int>(threadIdx.x & 63), i = min(lane_i, nbx * nby - 1);
+    const int by = i / nbx, bx = i - by * nbx;
+    auto off = [&](int s) { return (by + s % N) * PW + bx + s / N; };
+    auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
+    int value;
+    if constexpr (R >= 3 || AR || CH == 2) {
+      const int origin = by * PW + bx;
+      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE>(lane_i == i, sample, [&](int site) {
+        const float* t = tile + from_lane(origin, site);
+        return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
+      });
+      value = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
+    } else {
+      float ta, tb, td;
+      structure_tensor<N, true>(sample, ta, tb, td);
+      bool near = false;
+      const Bucket bk = hash_fast<RULE_LITE>(ta, tb, td, &near);
+      value = near && lane_i == i ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
+                                  : (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
+    }
+    if (lane_i == i) bucket[by * BX + bx] = value;
+  }
+}
+
 // One block per TX x TY output tile, one thread per output pixel (kZoomTiles).  (Kernels
 // without anti-ringing: at least 6 waves per SIMD, a register budget their out-of-line
 // re-decision inherits; r2 anti-ringing kernels and r3 ones on 16 x 16 tiles: 5, at most 96
@@ -277,32 +315,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   stage_used<P, PH, PW, TX * TY, AR>(tile, pw, in, io.in_dt, io.in_max, io.in_rmax, io.in_pitch, io.in_cstride, io.W, io.H,
                             bx0 - (R - 1), by0 - (R - 1), nbx + N - 1, nby + N - 1);
   __syncthreads();
-  // hash every base pixel the tile's outputs use (unclamped LUT row: bucket 9-row blocks
-  // are clamped per texel by the bilinear fetch, as the sampler does)
-  // (whole waves: the re-decision takes all lanes; those past the last base pixel repeat it)
-  for (int i0 = threadIdx.x & ~63; i0 < nbx * nby; i0 += TX * TY) {
-    const int lane_i = i0 + static_cast<int>(threadIdx.x & 63), i = min(lane_i, nbx * nby - 1);
-    const int by = i / nbx, bx = i - by * nbx;
-    auto off = [&](int s) { return (by + s % N) * PW + bx + s / N; };
-    auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
-    int value;
-    if constexpr (R >= 3 || AR || CH == 2) {
-      const int origin = by * PW + bx;
-      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE>(lane_i == i, sample, [&](int site) {
-        const float* t = tile + from_lane(origin, site);
-        return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
-      });
-      value = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
-    } else {
-      float ta, tb, td;
-      structure_tensor<N, true>(sample, ta, tb, td);
-      bool near = false;
-      const Bucket bk = hash_fast<RULE_LITE>(ta, tb, td, &near);
-      value = near && lane_i == i ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
-                                  : (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
-    }
-    if (lane_i == i) bucket[by * BX + bx] = value;
-  }
+  hash_bases<R, AR, CH, TAB, BX, PW, PN, TX * TY>(tile, bucket, nbx, nby);
   __syncthreads();
 
   const int ox = ox0 + threadIdx.x % TX, oy = oy0 + threadIdx.x / TX;
@@ -409,13 +422,133 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   for (int c = 0; c < P; ++c) {
     float v = res[c];
     if (AR) {
-      const float h = hi2[c] * __builtin_amdgcn_rcpf(hi[c]) - 0.1f, l = 1.1f - lo2[c] * __builtin_amdgcn_rcpf(lo[c]);
-      const float cl = fminf(fmaxf(v, l), h);
-      v = v * (1.0f - 0.8f) + cl * 0.8f;  // mix(res, clamp(res, lo, hi), 0.8), no final clamp
+      v = zoom_ring(v, hi[c], lo[c], hi2[c], lo2[c]);
     } else {
       v = fminf(fmaxf(v, 0.f), 1.f);
     }
     store_elem(ob + c * io.out_cstride * esz_out, static_cast<int64_t>(oy) * io.out_pitch + ox, io.out_dt, v);
+  }
+}
+
+// The same for plans that scale the width by exactly 2 (and have the weight table): outputs 2k + 1
+// and 2k + 2 share base pixel k, so a thread takes both and reads the window's samples and
+// powers from LDS once for the two (TX base pixels x TY output rows per block; k = -1 ..
+// in_w - 1, the first and the last with one output each).  Sums run in the same order.
+// One output per thread read 1.07 KB of LDS per output for AR rgb (154 of its 287 us) beside a
+// VALU share that overlapped it badly; this form is bound by VALU issue.  4 x 720p -> 1440p,
+// one output -> two: r2 113 -> 75 us, r2-yuv 146 -> 98, r3 129 -> 101, r3-rgb 207 -> 153, ar-r2
+// 196 -> 133, ar-r2-yuv 303 -> 211, ar-r2-rgb 279 -> 211; 640 x 360 -> 1280 x 720 ar-r2 22.5 -> 19.7.
+// 256 threads per block: 512 gave 249 us for ar-r2-rgb (waits at its two barriers), 128 gave 220.
+template <int R, bool AR, int CH, int TX, int TY>
+__global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const float4* __restrict__ wtab, int nphy,
+                                                                 const int4* __restrict__ phase, int out_w,
+                                                                 int out_h) {
+  constexpr int P = CH == 0 ? 1 : 3;
+  constexpr int N = 2 * R, HALF = N * N / 2, GROUPS = (HALF + 3) / 4;
+  constexpr int BX = TX, BY = TY + 1;
+  constexpr int PW = BX + N - 1, PH = BY + N - 1, PN = PW * PH;
+  constexpr int NT = AR ? 4 : 2;
+  __shared__ float tile[P * PN];
+  __shared__ int bucket[BY * BX];
+  __shared__ float4 pw[AR ? P * PN : 1];
+
+  const BlockXYZ bk3 = block_xyz((io.W + 1 + TX - 1) / TX, (out_h + TY - 1) / TY, io.batch);
+  const int f = bk3.z;
+  const int bx0 = bk3.x * TX - 1, oy0 = bk3.y * TY;
+  const int4* phy_tab = phase + out_w;
+  const int by0 = phy_tab[oy0].x;
+  const int nbx = min(TX, io.W - bx0);
+  const int nby = phy_tab[min(oy0 + TY, out_h) - 1].x - by0 + 1;
+  stage_used<P, PH, PW, TX * TY, AR>(tile, pw, frame_in(io, f), io.in_dt, io.in_max, io.in_rmax, io.in_pitch,
+                                     io.in_cstride, io.W, io.H, bx0 - (R - 1), by0 - (R - 1), nbx + N - 1,
+                                     nby + N - 1);
+  __syncthreads();
+  hash_bases<R, AR, CH, true, BX, PW, PN, TX * TY>(tile, bucket, nbx, nby);
+  __syncthreads();
+
+  const int lbx = threadIdx.x % TX, oy = oy0 + threadIdx.x / TX;
+  if (lbx >= nbx || oy >= out_h) return;
+  const int ox = 2 * (bx0 + lbx) + 1;  // this thread's outputs: ox (phase index 1), ox + 1 (phase index 0)
+  const bool first = ox >= 0, second = ox + 1 < out_w;
+  const int4 phy = phy_tab[oy];
+  const int lby = phy.x - by0;
+  const int row = bucket[lby * BX + lbx];
+  if (io.buckets) {
+    int32_t* b = io.buckets + f * io.bucket_bstride + static_cast<int64_t>(oy) * out_w + ox;
+    if (first) b[0] = row;
+    if (second) b[1] = row;
+  }
+  const int trow = min(max(row, kZoomRowLo), kZoomRowLo + kZoomRows - 1) - kZoomRowLo;
+  const float4* wt[2];
+  wt[1] = wtab + static_cast<int64_t>((trow * nphy + phy.z) * 2) * (GROUPS * NT);
+  wt[0] = wt[1] + GROUPS * NT;
+  const float* tp = tile + lby * PW + lbx;
+  const float4* pp = pw + lby * PW + lbx;
+  float res[2][P], hi[2][P], lo[2][P], hi2[2][P], lo2[2][P];
+#pragma unroll
+  for (int o = 0; o < 2; ++o)
+#pragma unroll
+    for (int c = 0; c < P; ++c) res[o][c] = hi[o][c] = lo[o][c] = hi2[o][c] = lo2[o][c] = 0.f;
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    __builtin_amdgcn_sched_barrier(0);  // one group's weights live at a time
+    float4 w4[2][NT];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) w4[o][j] = wt[o][g * NT + j];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int p = 4 * g + k;
+      if (p >= HALF) continue;
+      if (AR) __builtin_amdgcn_sched_barrier(0);  // one tap pair's samples and powers live at a time
+      const int q = N * N - 1 - p;
+      const int ip = p % N * PW + p / N, iq = q % N * PW + q / N;
+#pragma unroll
+      for (int c = 0; c < P; ++c) {
+        const float lp = tp[c * PN + ip], lq = tp[c * PN + iq];
+        float4 a, b;
+        if (AR) {
+          a = pp[c * PN + ip];
+          b = pp[c * PN + iq];
+        }
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+          auto w = [&](int j) { return k == 0 ? w4[o][j].x : (k == 1 ? w4[o][j].y : (k == 2 ? w4[o][j].z : w4[o][j].w)); };
+          res[o][c] = fmaf(lq, w(1), fmaf(lp, w(0), res[o][c]));
+          if constexpr (AR) {
+            hi[o][c] = fmaf(b.x, w(3), fmaf(a.x, w(2), hi[o][c]));
+            lo[o][c] = fmaf(b.y, w(3), fmaf(a.y, w(2), lo[o][c]));
+            hi2[o][c] = fmaf(b.z, w(3), fmaf(a.z, w(2), hi2[o][c]));
+            lo2[o][c] = fmaf(b.w, w(3), fmaf(a.w, w(2), lo2[o][c]));
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int c = 0; c < P; ++c) {
+        asm volatile("" : "+v"(res[o][c]));
+        if (AR) asm volatile("" : "+v"(hi[o][c]), "+v"(lo[o][c]), "+v"(hi2[o][c]), "+v"(lo2[o][c]));
+      }
+  }
+  const int esz_out = elem_bytes(io.out_dt);
+  char* ob = static_cast<char*>(frame_out(io, f));
+#pragma unroll
+  for (int c = 0; c < P; ++c) {
+    float v[2];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+      v[o] = AR ? zoom_ring(res[o][c], hi[o][c], lo[o][c], hi2[o][c], lo2[o][c]) : fminf(fmaxf(res[o][c], 0.f), 1.f);
+    void* dst = ob + c * io.out_cstride * esz_out;
+    const int64_t at = static_cast<int64_t>(oy) * io.out_pitch + ox;
+    if (first && second) {
+      store_pair(dst, at, io.out_dt, v[0], v[1]);
+    } else {
+      if (first) store_elem(dst, at, io.out_dt, v[0]);
+      if (second) store_elem(dst, at + 1, io.out_dt, v[1]);
+    }
   }
 }
 
@@ -425,9 +558,16 @@ static hipError_t launch_zoom_tile(int r, bool ar, int channels, const Io& io, c
   constexpr int TX = kZoomTiles[T].w, TY = kZoomTiles[T].h;
   const dim3 grid(((out_w + TX - 1) / TX) * ((out_h + TY - 1) / TY) * io.batch), block(TX * TY);
   const float4* wtab = reinterpret_cast<const float4*>(zp.wtab);
+  // Width scaled by exactly 2 (any height whose phases fit the table): two outputs per thread,
+  // faster for every variant from 640 x 360 up (the kernel's comment has the figures).
+  const bool pair = zp.wtab && zp.nphx == 2 && out_w == 2 * io.W;
+  const dim3 pairs(((io.W + TX) / TX) * ((out_h + TY - 1) / TY) * io.batch);
 #define MPX_ZOOM(R, A, CH)                                                                                   \
   if (r == R && ar == A && channels == CH) {                                                                 \
-    if (zp.wtab)                                                                                             \
+    if (pair)                                                                                                \
+      hipLaunchKernelGGL((ravu_zoom_pair_kernel<R, A, CH, TX, TY>), pairs, block, 0, st, io, wtab, zp.nphy,  \
+                         zp.phase, out_w, out_h);                                                            \
+    else if (zp.wtab)                                                                                        \
       hipLaunchKernelGGL((ravu_zoom_kernel<R, A, CH, true, TX, TY>), grid, block, 0, st, io, lut, lut_ar, wtab, \
                          zp.nphx, zp.nphy, zp.phase, out_w, out_h);                                          \
     else                                                                                                     \
