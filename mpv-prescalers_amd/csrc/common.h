@@ -609,9 +609,7 @@ __device__ __attribute__((noinline)) Bucket hash_fp64(double a, double b, double
 // Bound by the latency of the wave that takes it, which holds its block's LDS meanwhile: one
 // lane's serial evaluation (up to 36 points of two five-point derivatives, r4 rgb luma in FP64
 // per sample) took 10-20 us where a wave otherwise lives about 10 (ravu-r4-rgb 640x360 51.6 us,
-// 21.2 with the path switched off; with the shared one 28.7).  It also costs the kernel fewer
-// registers: zoom-ar-r2-rgb 96 VGPRs and scratch -> 81 and none, 4 x 720p -> 1440p 340.4 ->
-// 288.9 us.  Small central-difference windows (lite, 3x) keep a lane's own evaluation: several
+// 21.2 with the path switched off; with the shared one 28.7).  Small central-difference windows (lite, 3x) keep a lane's own evaluation: several
 // of their lanes are near at once (lite-r2 8 x 1080p 126 us, shared 150).
 template <int N, bool FIVE, typename At>
 __device__ __forceinline__ void wave_tensor(uint64_t mask, At at, double& a, double& b, double& d) {
@@ -663,19 +661,45 @@ __device__ __forceinline__ void wave_tensor(uint64_t mask, At at, double& a, dou
   }
 }
 
-// The FP64 re-decision of the lanes whose FP32 decision is near a boundary (see wave_tensor).
-template <int N, bool FIVE, int RULE, typename At>
-__device__ __forceinline__ void redecide(bool near, At at, Bucket& bk) {
-  const uint64_t mask = __ballot(near);
-  if (mask) {
-    double a = 0.0, b = 0.0, d = 0.0;
-    wave_tensor<N, FIVE>(mask, at, a, b, d);
-    if (near) bk = hash_fp64<RULE>(a, b, d);
-  }
-}
-
 // Value of lane `i` (uniform) in every lane.
 __device__ __forceinline__ int from_lane(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
+
+// SITES of redecide: an rgb sample is the FP64 luma of three, which makes a lane's own evaluation
+// dear (ravu-r4-rgb 640x360: 26.5 us with 1 or 2, 39.6 with 0; a frame of isolated dots
+// 1280x720 88 us with 1, 81 with 2); elsewhere one turn is still cheaper than a lane alone (ravu-r4
+// 1280x720 36.5 against 40.9), two turns are not (r3, isolated dots: 37.0 with 1, 39.1 with 2, 39 to
+// 41 with 4 to 16).
+constexpr int wave_sites(int channels) { return channels == 2 ? 2 : 1; }
+
+// One lane's own evaluation and hash, out of line: inlined, its registers (the double atan2 alone
+// takes 56) would set the occupancy of every wave.  `sample(X, Y)` comes by value, and each
+// kernel's accessor is a type of its own, so each has its own instance, with its caller's
+// register budget (the lean tensor form keeps it from spilling).
+template <int N, bool FIVE, int RULE, typename Sample>
+__device__ __attribute__((noinline)) Bucket redecide_alone(Sample sample) {
+  double a, b, d;
+  structure_tensor_fp64<N, FIVE, true>([&](int i) { return sample(i / N, i % N); }, a, b, d);
+  return hash_reference<RULE, double>(a, b, d);
+}
+
+// The FP64 re-decision of the lanes whose FP32 decision is near a boundary.  `at(o)` gives the
+// accessor (X, Y) -> sample of the window at offset o, of which `o` is this lane's.
+// Up to SITES near lanes are taken one after the other by the whole wave (wave_tensor, which also
+// says what bounds it); more evaluate their own windows at the same time.  A wave full of near
+// sites (a frame of 45-degree stripes) would take 64 turns: ravu-r4 1280x720 1512 us, against 170
+// with each lane on its own.
+template <int N, bool FIVE, int RULE, int SITES, typename At>
+__device__ __forceinline__ void redecide(bool near, int o, At at, Bucket& bk) {
+  const uint64_t mask = __ballot(near);
+  if (!mask) return;
+  if (__popcll(mask) <= SITES) {
+    double a = 0.0, b = 0.0, d = 0.0;
+    wave_tensor<N, FIVE>(mask, [&](int site) { return at(from_lane(o, site)); }, a, b, d);
+    if (near) bk = hash_fp64<RULE>(a, b, d);
+  } else if (near) {
+    bk = redecide_alone<N, FIVE, RULE>(at(o));
+  }
+}
 
 // Hash of one site: FP32, re-decided in FP64 when near a boundary.  getf(i) -> float
 // and getd(i) -> double return window sample i (getd widens the same stored values, and
@@ -694,17 +718,17 @@ __device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
   return bk;
 }
 
-// The same with the wave's shared re-decision (wave_tensor).  getf(i) returns
-// window sample i; at(site): see wave_tensor.  All lanes of the wave call it together; lanes
+// The same with the wave's shared re-decision.  getf(i) returns
+// window sample i; o, at: see redecide.  All lanes of the wave call it together; lanes
 // without a site (`valid` false) read their window too (inside the staged tile) but are never
 // re-decided.
-template <int N, bool FIVE, int RULE, typename GetF, typename At>
-__device__ __forceinline__ Bucket ravu_hash_wave(bool valid, GetF getf, At at) {
+template <int N, bool FIVE, int RULE, int SITES, typename GetF, typename At>
+__device__ __forceinline__ Bucket ravu_hash_wave(bool valid, GetF getf, int o, At at) {
   float a, b, d;
   structure_tensor<N, FIVE>(getf, a, b, d);
   bool near = false;
   Bucket bk = hash_fast<RULE>(a, b, d, &near);
-  redecide<N, FIVE, RULE>(near && valid, at, bk);
+  redecide<N, FIVE, RULE, SITES>(near && valid, o, at, bk);
   return bk;
 }
 

@@ -93,8 +93,8 @@ template <int N, int CH, int PW, int PN>
 __device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
   auto sample = [&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); };
   if constexpr (wave_redecide<CH>()) {
-    return ravu_hash_wave<N, true, RULE_LOG2>(valid, sample, [&](int site) {
-      const float* w = t + from_lane(o, site);
+    return ravu_hash_wave<N, true, RULE_LOG2, wave_sites(CH)>(valid, sample, o, [&](int at) {
+      const float* w = t + at;
       return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
     });
   } else {
@@ -313,6 +313,17 @@ __device__ __host__ constexpr int lat2x(int X, int Y) { return STEP == 2 ? X + Y
 template <int N, int STEP>
 __device__ __host__ constexpr int lat2y(int X, int Y) { return STEP == 2 ? Y - X : Y - X + 1; }
 
+// FP64 samples of a step 2 / 3 window from the staged input at t = the site's (px and py have
+// the same parity; the int11 tile follows the input's).
+template <int N, int STEP, int CH, int PW, int PN>
+struct LatticeWindow {
+  const float* t;
+  __device__ __forceinline__ double operator()(int X, int Y) const {
+    const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
+    return luma_d<CH>(t, (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
+  }
+};
+
 // One site's step 2 (int10, STEP = 2) or step 3 (int01, STEP = 3) on the lattice, and
 // the combine for one output row: STEP 2 writes row 2y = (input, int10) pairs, STEP 3
 // row 2y+1 = (int01, int11) pairs (ravu-r3.hook:426-437), so each step stores contiguous
@@ -331,12 +342,8 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
   auto sample = [&](int i) { return luma_f<CH>(src(i), 0, PN); };
   Bucket bk;
   if constexpr (wave_redecide<CH>()) {
-    bk = ravu_hash_wave<N, true, RULE_LOG2>(valid, sample, [&](int site) {
-      const int o = from_lane(base, site);
-      return [hk, o](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
-        const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
-        return luma_d<CH>(hk, o + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
-      };
+    bk = ravu_hash_wave<N, true, RULE_LOG2, wave_sites(CH)>(valid, sample, base, [&](int o) {
+      return LatticeWindow<N, STEP, CH, PW, PN>{hk + o};
     });
   } else {
     bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return luma_d<CH>(src(i), 0, PN); });
@@ -552,8 +559,8 @@ __global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))
     Sep::site([&](bool five, int i) { return five ? tf[e + i] : tc[e + i]; }, [&](int i) { return td[e + i]; }, a, b, d);
     bool near = false;
     Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
-    redecide<N, true, RULE_LOG2>(near && valid && (s == 0 || second), [&](int site) {
-      const float* w = tile + from_lane(o, site) + s * PW;
+    redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid && (s == 0 || second), o, [&](int at) {
+      const float* w = tile + at + s * PW;
       return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
     }, bk);
     row[s] = bucket_row<RULE_LOG2>(bk, 648);
@@ -683,13 +690,12 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
         [&](int i) { return td[entry(i + 1 - s)]; }, a, b, d);
     bool near = false;
     Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
-    redecide<N, true, RULE_LOG2>(near && valid, [&](int site) {
-      const int o = from_lane(base, site);
-      return [hk, o, s](int X, int Y) {  // (px and py have the same parity; the int11 tile follows the input's)
-        const int px = X - s + Y - N + 2, py = Y - X + s;
-        return luma_d<CH>(hk, o + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
-      };
-    }, bk);
+    if (s == 0)
+      redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
+                                   [&](int o) { return LatticeWindow<N, 2, CH, PW, PN>{hk + o}; }, bk);
+    else
+      redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
+                                   [&](int o) { return LatticeWindow<N, 3, CH, PW, PN>{hk + o}; }, bk);
     row[s] = bucket_row<RULE_LOG2>(bk, 648);
     if (io.buckets && valid)
       io.buckets[f * io.bucket_bstride + (s + 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row[s];

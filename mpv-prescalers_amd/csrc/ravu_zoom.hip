@@ -113,21 +113,6 @@ __device__ __forceinline__ double zluma_d(const float* t, int o, int n) {
   return static_cast<double>(t[o]);
 }
 
-// FP64 re-decision of one base pixel's hash, out of line (the kernels without anti-ringing):
-// it runs for a small fraction of sites, and inlined its registers (the double atan2 alone
-// takes 56) would set the occupancy of every wave (zoom-r2: 96 -> 51 VGPRs, r3 rgb: 137 ->
-// 61).  Its register budget follows its callers' (6 waves per SIMD, below), so the lean
-// tensor form keeps it from spilling.  `t` is the staged tile, `o` the window's first sample.
-// (one instance per calling kernel, TAB, so each inherits its own caller's budget)
-template <int N, int CH, int PW, int PN, bool TAB>
-__device__ __attribute__((noinline)) int zoom_redecide(const float* t, int o) {
-  double a, b, d;
-  structure_tensor_fp64<N, true, true>([&](int s) { return zluma_d<CH>(t, o + (s % N) * PW + s / N, PN); },
-                                          a, b, d);
-  const Bucket bk = hash_reference<RULE_LITE, double>(a, b, d);
-  return (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
-}
-
 // Stage the part of the PH x PW staging area that a tile's outputs read: the uh x uw
 // samples per plane around its base pixels (at 2x 8 x 20 of 12 x 36), clamp-to-edge, at
 // the area's row stride PW.  AR forms store each sample's anti-ringing powers beside it
@@ -250,6 +235,9 @@ __device__ __forceinline__ float zoom_ring(float v, float hi, float lo, float hi
 
 // Hash every base pixel of a tile (nbx x nby) into bucket[by * BX + bx]: the unclamped LUT row
 // (bucket 9-row blocks are clamped per texel by the bilinear fetch, as the sampler does).
+// r2's near lanes evaluate their own windows (16 points: a turn of the wave is no cheaper, and the
+// kernel is smaller: zoom-ar-r2-rgb 4 x 720p -> 1440p 210 -> 204 us, ar-r2 134 -> 127).  TAB only
+// tells the kernels apart: the out-of-line evaluation follows its caller's register budget.
 template <int R, bool AR, int CH, bool TAB, int BX, int PW, int PN, int NT>
 __device__ __forceinline__ void hash_bases(const float* tile, int* bucket, int nbx, int nby) {
   constexpr int N = 2 * R;
@@ -259,23 +247,12 @@ __device__ __forceinline__ void hash_bases(const float* tile, int* bucket, int n
     const int by = i / nbx, bx = i - by * nbx;
     auto off = [&](int s) { return (by + s % N) * PW + bx + s / N; };
     auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
-    int value;
-    if constexpr (R >= 3 || AR || CH == 2) {
-      const int origin = by * PW + bx;
-      const Bucket bk = ravu_hash_wave<N, true, RULE_LITE>(lane_i == i, sample, [&](int site) {
-        const float* t = tile + from_lane(origin, site);
-        return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
-      });
-      value = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
-    } else {
-      float ta, tb, td;
-      structure_tensor<N, true>(sample, ta, tb, td);
-      bool near = false;
-      const Bucket bk = hash_fast<RULE_LITE>(ta, tb, td, &near);
-      value = near && lane_i == i ? zoom_redecide<N, CH, PW, PN, TAB>(tile, off(0))
-                                  : (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
-    }
-    if (lane_i == i) bucket[by * BX + bx] = value;
+    const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, R == 2 ? 0 : wave_sites(CH)>(
+        lane_i == i, sample, by * PW + bx, [&](int o) {
+          const float* t = tile + o;
+          return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
+        });
+    if (lane_i == i) bucket[by * BX + bx] = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
   }
 }
 
