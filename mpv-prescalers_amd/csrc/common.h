@@ -671,6 +671,19 @@ __device__ __forceinline__ int from_lane(int v, int i) { return __builtin_amdgcn
 // 41 with 4 to 16).
 constexpr int wave_sites(int channels) { return channels == 2 ? 2 : 1; }
 
+// A staged tile as an accessor carries it into that function: an LDS pointer, as a generic one's
+// reads are flat loads there (45-degree
+// stripes 1280x720: ravu-r4 170 -> 133 us, r3 87 -> 82).  Not for rgb, where the compiler
+// then keeps so many samples at hand that r4's kernels lose a wave per SIMD (134 VGPRs).
+template <int CH>
+struct TilePointer {
+  typedef const __attribute__((address_space(3))) float* T;
+};
+template <>
+struct TilePointer<2> {
+  typedef const float* T;
+};
+
 // One lane's own evaluation and hash, out of line: inlined, its registers (the double atan2 alone
 // takes 56) would set the occupancy of every wave.  `sample(X, Y)` comes by value, and each
 // kernel's accessor is a type of its own, so each has its own instance, with its caller's
@@ -686,7 +699,7 @@ __device__ __attribute__((noinline)) Bucket redecide_alone(Sample sample) {
 // accessor (X, Y) -> sample of the window at offset o, of which `o` is this lane's.
 // Up to SITES near lanes are taken one after the other by the whole wave (wave_tensor, which also
 // says what bounds it); more evaluate their own windows at the same time.  A wave full of near
-// sites (a frame of 45-degree stripes) would take 64 turns: ravu-r4 1280x720 1512 us, against 170
+// sites (a frame of 45-degree stripes) would take 64 turns: ravu-r4 1280x720 1512 us, against 133
 // with each lane on its own.
 template <int N, bool FIVE, int RULE, int SITES, typename At>
 __device__ __forceinline__ void redecide(bool near, int o, At at, Bucket& bk) {

@@ -51,12 +51,13 @@ constexpr TileShape kLiteTiles[] = {{32, 8}, {64, 4}, {32, 4}};
 constexpr TileShape k3xTiles[] = {{32, 8}, {64, 4}};
 constexpr TileShape kRavuTiles[] = {{32, 8}, {32, 16}, {64, 8}};
 constexpr TileShape kZoomTiles[] = {{32, 8}, {16, 16}};
-// Full RAVU r3 has its shapes in another order, its fastest first: 64 x 8 for luma and yuv (r3
-// 1366x768 32.0 us, 32 x 8 34.8, 32 x 16 33.9; 4 x 1080p 159.4, 162.3, 163.7), 32 x 16 for rgb, whose
-// fourth plane of 64 x 8 tiles leaves two blocks per compute unit (2 x 1080p 140.4 us, 32 x 8
-// 150.5, 64 x 8 169.5).  r4 is faster on 32 x 8 (r4-yuv 195.9 us, 205.9, 204.8).
+// Full RAVU r3's yuv and rgb forms have their shapes in another order, the fastest first: 64 x 8
+// for yuv (4 x 1080p 251.7 us, 32 x 8 264.4, 32 x 16 249.5; 640x360 20.3, 21.3, 20.4), 32 x 16 for
+// rgb, whose fourth plane of 64 x 8 tiles leaves two blocks per compute unit (2 x 1080p 140.4 us,
+// 32 x 8 150.5, 64 x 8 169.5).  r3 luma is fastest on 32 x 8 (4 x 1080p 162.0, 64 x 8 167.5, 32 x 16
+// 173.0), and so is r4 (r4-yuv 195.9 us, 205.9, 204.8).
 constexpr int ravu_tile_index(int r, int channels, int tile) {
-  if (r != 3) return tile;
+  if (r != 3 || channels == 0) return tile;
   if (channels == 2) return tile < 2 ? 1 - tile : tile;
   return (tile + 2) % 3;
 }

@@ -313,14 +313,19 @@ __device__ __host__ constexpr int lat2x(int X, int Y) { return STEP == 2 ? X + Y
 template <int N, int STEP>
 __device__ __host__ constexpr int lat2y(int X, int Y) { return STEP == 2 ? Y - X : Y - X + 1; }
 
-// FP64 samples of a step 2 / 3 window from the staged input at t = the site's (px and py have
-// the same parity; the int11 tile follows the input's).
+// FP64 samples of a step 2 / 3 window, `at` = LDS offset of the site in the staged input (px and
+// py have the same parity; the int11 tile follows the input's).  It keeps the window's lowest
+// address, so the reads' offsets are non-negative immediates (otherwise the addresses are
+// registers of their own).
 template <int N, int STEP, int CH, int PW, int PN>
 struct LatticeWindow {
-  const float* t;
+  static constexpr int LOW = N / 2 * (PW + 1);
+  typename TilePointer<CH>::T t;
+  __device__ __forceinline__ LatticeWindow(const float* hk, int at)
+      : t((typename TilePointer<CH>::T)(hk + at - LOW)) {}
   __device__ __forceinline__ double operator()(int X, int Y) const {
     const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
-    return luma_d<CH>(t, (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
+    return luma_d<CH>((const float*)t, LOW + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
   }
 };
 
@@ -343,7 +348,7 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
   Bucket bk;
   if constexpr (wave_redecide<CH>()) {
     bk = ravu_hash_wave<N, true, RULE_LOG2, wave_sites(CH)>(valid, sample, base, [&](int o) {
-      return LatticeWindow<N, STEP, CH, PW, PN>{hk + o};
+      return LatticeWindow<N, STEP, CH, PW, PN>(hk, o);
     });
   } else {
     bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return luma_d<CH>(src(i), 0, PN); });
@@ -560,8 +565,8 @@ __global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))
     bool near = false;
     Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
     redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid && (s == 0 || second), o, [&](int at) {
-      const float* w = tile + at + s * PW;
-      return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
+      const auto w = (typename TilePointer<CH>::T)(tile + at + s * PW);
+      return [w](int X, int Y) { return luma_d<CH>((const float*)w, Y * PW + X, PN); };
     }, bk);
     row[s] = bucket_row<RULE_LOG2>(bk, 648);
     if (io.buckets && valid && (s == 0 || second))
@@ -692,10 +697,10 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
     Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
     if (s == 0)
       redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
-                                   [&](int o) { return LatticeWindow<N, 2, CH, PW, PN>{hk + o}; }, bk);
+                                   [&](int o) { return LatticeWindow<N, 2, CH, PW, PN>(hk, o); }, bk);
     else
       redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
-                                   [&](int o) { return LatticeWindow<N, 3, CH, PW, PN>{hk + o}; }, bk);
+                                   [&](int o) { return LatticeWindow<N, 3, CH, PW, PN>(hk, o); }, bk);
     row[s] = bucket_row<RULE_LOG2>(bk, 648);
     if (io.buckets && valid)
       io.buckets[f * io.bucket_bstride + (s + 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row[s];

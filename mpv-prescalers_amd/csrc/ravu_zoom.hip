@@ -249,8 +249,8 @@ __device__ __forceinline__ void hash_bases(const float* tile, int* bucket, int n
     auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
     const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, R == 2 ? 0 : wave_sites(CH)>(
         lane_i == i, sample, by * PW + bx, [&](int o) {
-          const float* t = tile + o;
-          return [t](int X, int Y) { return zluma_d<CH>(t, Y * PW + X, PN); };
+          const auto t = (typename TilePointer<CH>::T)(tile + o);
+          return [t](int X, int Y) { return zluma_d<CH>((const float*)t, Y * PW + X, PN); };
         });
     if (lane_i == i) bucket[by * BX + bx] = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
   }
