@@ -415,6 +415,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
 // VALU share that overlapped it badly; this form is bound by VALU issue.  4 x 720p -> 1440p,
 // one output -> two: r2 113 -> 75 us, r2-yuv 146 -> 98, r3 129 -> 101, r3-rgb 207 -> 153, ar-r2
 // 196 -> 133, ar-r2-yuv 303 -> 211, ar-r2-rgb 279 -> 211; 640 x 360 -> 1280 x 720 ar-r2 22.5 -> 19.7.
+// (r2's re-decision by each lane came after: ar-r2 126, ar-r2-rgb 204, r2-rgb 2 x 720p at 1.5x 51.)
 // 256 threads per block: 512 gave 249 us for ar-r2-rgb (waits at its two barriers), 128 gave 220.
 template <int R, bool AR, int CH, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const float4* __restrict__ wtab, int nphy,
