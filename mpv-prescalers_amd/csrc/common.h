@@ -381,12 +381,45 @@ template <int N, bool FIVE>
 __device__ __host__ constexpr double deriv_scale(int p) {
   return (p == 0 || p == N - 1) ? 1.0 : (FIVE && p >= 2 && p + 2 <= N - 1) ? 1.0 / 12.0 : 0.5;
 }
+// The sample that a hash sees: plane 0's, or for rgb (CH = 2) the BT.709 luma in FP64.  A luma
+// rounded to FP32 first would be off by 1e-7, in faint detail 1e-5 to 1e-3 of the derivative and
+// outside every margin of hash_fast; the difference of FP64 lumas, rounded once, is as good as
+// that of two FP32 samples.
+// Bound by VALU issue: an FP64 difference and its conversion take the time of four FP32
+// instructions (ordinary frames, FP32 luma -> FP64: r2-rgb 2 x 1080p 115 -> 129 us, r3-rgb 142 -> 155,
+// r4-rgb 214 -> 231, zoom-ar-r2-rgb 720p -> 1440p 57.4 -> 56.0), while a re-decision reads one
+// sample instead of three and no longer computes their luma (45-degree stripes 1280x720: r4-rgb
+// 386 -> 116, r3-rgb 159 -> 74, zoom-r3-rgb at 1.5x 142 -> 58; large flat shapes: r4-rgb 145 -> 100).
+template <int CH> struct HashSampleOf { typedef float T; };
+template <> struct HashSampleOf<2> { typedef double T; };
+template <int CH>
+using HashSample = typename HashSampleOf<CH>::T;
+// (the oracle's operations in its order)
+__device__ __forceinline__ double luma709(float r, float g, float b) {
+#pragma clang fp contract(off)
+  return 0.2126 * static_cast<double>(r) + 0.7152 * static_cast<double>(g) + 0.0722 * static_cast<double>(b);
+}
+// Lumas of `count` staged samples (rounded up to pairs; n samples per plane, even; both arrays 16-byte
+// aligned) by the block's NT threads.
+template <int NT>
+__device__ __forceinline__ void fill_luma(const float* t, double* luma, int n, int count) {
+  const float2* s = reinterpret_cast<const float2*>(t);
+  for (int i = threadIdx.x; 2 * i < count; i += NT) {
+    const float2 r = s[i], g = s[n / 2 + i], b = s[n + i];
+    reinterpret_cast<double2*>(luma)[i] = make_double2(luma709(r.x, g.x, b.x), luma709(r.y, g.y, b.y));
+  }
+}
+
+__device__ __forceinline__ float difference(float a, float b) { return a - b; }
+__device__ __forceinline__ float difference(double a, double b) { return static_cast<float>(a - b); }
 template <int N, bool FIVE, typename Line>
 __device__ __forceinline__ float deriv_unscaled(Line s, int p) {
-  if (p == 0) return s(1) - s(0);
-  if (p == N - 1) return s(N - 1) - s(N - 2);
-  if (FIVE && p >= 2 && p + 2 <= N - 1) return fmaf(8.0f, s(p + 1) - s(p - 1), s(p - 2) - s(p + 2));
-  return s(p + 1) - s(p - 1);
+#pragma clang fp contract(off)
+  if (p == 0) return difference(s(1), s(0));
+  if (p == N - 1) return difference(s(N - 1), s(N - 2));
+  if (FIVE && p >= 2 && p + 2 <= N - 1)
+    return fmaf(8.0f, difference(s(p + 1), s(p - 1)), difference(s(p - 2), s(p + 2)));
+  return difference(s(p + 1), s(p - 1));
 }
 
 // Gradient grid of an N x N window: positions P0 .. P1 - 1 on both axes.
@@ -403,15 +436,25 @@ struct GradGrid {
 // stencil scales folded into its Gaussian weight (compile-time constants); where gx and gy
 // carry the same scale one product w'*gx serves both a and b (lite-r3 8 x 1080p 132.4 ->
 // 128.4 us, zoom-r2 4 x 720p -> 1440p 117.1 -> 113.3).
+// FP64 samples of a 4 x 4 window (32 derivatives of 16 samples) are first rounded relative to an
+// inner one: with border derivatives in the grid no sample is far from it, and the rounding is
+// at most 6.6 u of the tensor's norm, where larger windows' may be any multiple.
 template <int N, bool FIVE, typename Get>
 __device__ __forceinline__ void structure_tensor(Get get, float& a, float& b, float& d) {
 #pragma clang fp contract(off)
   using GG = GradGrid<N>;
+  if constexpr (N == 4 && sizeof(get(0)) == 8) {
+    const double c = get(N + 1);
+    return structure_tensor<N, FIVE>([&](int i) { return static_cast<float>(get(i) - c); }, a, b, d);
+  }
   a = b = d = 0.f;
 #pragma unroll
   for (int X = GG::P0; X < GG::P1; ++X) {
+    // (FP64 samples: the columns that three derivatives need live at a time)
+    if constexpr (sizeof(get(0)) == 8) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int Y = GG::P0; Y < GG::P1; ++Y) {
+      if constexpr (sizeof(get(0)) == 8) __builtin_amdgcn_sched_barrier(0);
       const float gx = deriv_unscaled<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
       const float gy = deriv_unscaled<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
       const double cx = deriv_scale<N, FIVE>(X), cy = deriv_scale<N, FIVE>(Y);
@@ -516,12 +559,17 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 // (floor(log2 v)), and the angle atan2(L1 - a, b) in units of pi/24 is an odd degree-13
 // minimax polynomial of min / max (fitted by the Remez exchange; |error| <= 2.6e-6 units
 // in FP32).  Sets *near, and the caller re-decides in FP64, when a decision may differ from
-// the exact one.  The tensor's own FP32 error (u = 2^-24): 36 terms of five roundings summed
-// one after the other give a, d within 41 u of themselves and b within 41 u T / 2, hence
-// sqrt(L1) within a relative 41 u = 2.5e-6 (margin 3.8e-6), L2 within 41 u T (6.9e-6 T), mu
-// within 55 u at 1/4 and 92 u at 1/2 (6e-6), and the angle within 29 u T / (2 delta) (32 u,
-// plus 1e-5 units for the evaluation, whose error is below 5e-6).  Exact cases (flat window
-// T = 0, b = 0 exactly) are never near.
+// the exact one.  The tensor's own FP32 error (u = 2^-24): differences of exact samples are off by
+// u each, which the five-point stencil can amplify by cancellation, but never past 1.83 u of the
+// tensor's norm (the largest ratio over all 8 x 8 windows, an eigenvalue; 6 x 6: 1.69, central
+// and border stencils: 1); with the derivative's own rounding that is 6 u of a, d.  36 terms,
+// each squared and weighted, summed one after the other then give a, d within 44 u of themselves
+// and b within 44 u T / 2 (column sums, SepTensor: two levels of at most six terms and rounded
+// 1-D weights, 22 u), hence sqrt(L1) within a relative 44 u = 2.6e-6 (margin 3.8e-6), L2 within
+// 44 u T (6.9e-6 T = 115 u), mu within 59 u at 1/4 and 99 u at 1/2 (6e-6 = 100 u), and the angle
+// within 31 u T / (2 delta) (32 u, plus 1e-5 units for the evaluation, whose error is below
+// 5e-6).  A sample that is itself rounded, like an rgb luma in FP32, has no place in this bound:
+// see HashSample.  Exact cases (flat window T = 0, b = 0 exactly) are never near.
 // Bound by VALU issue: the exactly rounded sqrtf, the library atan2f and log2f that this
 // replaces took about 75 of a hash's ~150 instructions, and an angle margin of 2.4e-4 units
 // sent 3-4x as many sites to FP64.  Measured: ravu-r3 1366x768 44.3 -> 37.5 us, r4-yuv
@@ -607,9 +655,9 @@ __device__ __attribute__((noinline)) Bucket hash_fp64(double a, double b, double
 // `at(site)` gives an accessor (X, Y) -> sample of the window of lane `site`.  Every lane of
 // the wave must be active.  a, b, d are set in the lanes of `mask`.
 // Bound by the latency of the wave that takes it, which holds its block's LDS meanwhile: one
-// lane's serial evaluation (up to 36 points of two five-point derivatives, r4 rgb luma in FP64
-// per sample) took 10-20 us where a wave otherwise lives about 10 (ravu-r4-rgb 640x360 51.6 us,
-// 21.2 with the path switched off; with the shared one 28.7).  Small central-difference windows (lite, 3x) keep a lane's own evaluation: several
+// lane's serial evaluation (up to 36 points of two five-point derivatives, for r4 rgb of a luma
+// computed per sample) took 10-20 us where a wave otherwise lives about 10 (ravu-r4-rgb 640x360
+// 51.6 us, 21.2 with the path switched off; with the shared one 28.7).  Small central-difference windows (lite, 3x) keep a lane's own evaluation: several
 // of their lanes are near at once (lite-r2 8 x 1080p 126 us, shared 150).
 template <int N, bool FIVE, typename At>
 __device__ __forceinline__ void wave_tensor(uint64_t mask, At at, double& a, double& b, double& d) {
@@ -664,25 +712,18 @@ __device__ __forceinline__ void wave_tensor(uint64_t mask, At at, double& a, dou
 // Value of lane `i` (uniform) in every lane.
 __device__ __forceinline__ int from_lane(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
 
-// SITES of redecide: an rgb sample is the FP64 luma of three, which makes a lane's own evaluation
-// dear (ravu-r4-rgb 640x360: 26.5 us with 1 or 2, 39.6 with 0; a frame of isolated dots
-// 1280x720 88 us with 1, 81 with 2); elsewhere one turn is still cheaper than a lane alone (ravu-r4
-// 1280x720 36.5 against 40.9), two turns are not (r3, isolated dots: 37.0 with 1, 39.1 with 2, 39 to
-// 41 with 4 to 16).
-constexpr int wave_sites(int channels) { return channels == 2 ? 2 : 1; }
+// SITES of redecide: one turn of the wave is cheaper than a lane alone (ravu-r4 1280x720 36.5 us
+// against 40.9, r4-rgb 66.7 against 70.2), two turns are not (r3, isolated dots: 37.0 with 1, 39.1 with
+// 2, 39 to 41 with 4 to 16; r4-rgb, large flat shapes: 100.3 with 1, 102.6 with 2).
+constexpr int kWaveSites = 1;
 
-// A staged tile as an accessor carries it into that function: an LDS pointer, as a generic one's
-// reads are flat loads there (45-degree
-// stripes 1280x720: ravu-r4 170 -> 133 us, r3 87 -> 82).  Not for rgb, where the compiler
-// then keeps so many samples at hand that r4's kernels lose a wave per SIMD (134 VGPRs).
-template <int CH>
-struct TilePointer {
-  typedef const __attribute__((address_space(3))) float* T;
-};
-template <>
-struct TilePointer<2> {
-  typedef const float* T;
-};
+// The staged samples that a hash sees, as an accessor carries them into that function: an LDS
+// pointer, as a generic one's reads are flat loads there (45-degree stripes 1280x720: ravu-r4
+// 170 -> 133 us, r3 87 -> 82).
+template <typename T>
+using LdsSamples = const __attribute__((address_space(3))) T*;
+template <typename T>
+__device__ __forceinline__ LdsSamples<T> lds_samples(const T* p) { return (LdsSamples<T>)p; }
 
 // One lane's own evaluation and hash, out of line: inlined, its registers (the double atan2 alone
 // takes 56) would set the occupancy of every wave.  `sample(X, Y)` comes by value, and each
@@ -714,9 +755,9 @@ __device__ __forceinline__ void redecide(bool near, int o, At at, Bucket& bk) {
   }
 }
 
-// Hash of one site: FP32, re-decided in FP64 when near a boundary.  getf(i) -> float
-// and getd(i) -> double return window sample i (getd widens the same stored values, and
-// for RGB forms it recomputes the BT.709 luma in FP64).  LEAN picks the tensor forms.
+// Hash of one site: FP32, re-decided in FP64 when near a boundary.  getf(i) -> float or double
+// and getd(i) -> double return window sample i (for rgb both are the FP64 luma).  LEAN picks
+// the FP64 tensor's form.
 template <int N, bool FIVE, int RULE, bool LEAN = false, typename GetF, typename GetD>
 __device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
   float a, b, d;

@@ -51,15 +51,14 @@ constexpr TileShape kLiteTiles[] = {{32, 8}, {64, 4}, {32, 4}};
 constexpr TileShape k3xTiles[] = {{32, 8}, {64, 4}};
 constexpr TileShape kRavuTiles[] = {{32, 8}, {32, 16}, {64, 8}};
 constexpr TileShape kZoomTiles[] = {{32, 8}, {16, 16}};
-// Full RAVU r3's yuv and rgb forms have their shapes in another order, the fastest first: 64 x 8
-// for yuv (4 x 1080p 251.7 us, 32 x 8 264.4, 32 x 16 249.5; 640x360 20.3, 21.3, 20.4), 32 x 16 for
-// rgb, whose fourth plane of 64 x 8 tiles leaves two blocks per compute unit (2 x 1080p 140.4 us,
-// 32 x 8 150.5, 64 x 8 169.5).  r3 luma is fastest on 32 x 8 (4 x 1080p 162.0, 64 x 8 167.5, 32 x 16
-// 173.0), and so is r4 (r4-yuv 195.9 us, 205.9, 204.8).
+// Full RAVU's shapes in the order of each form, the fastest first.  luma and yuv: r3 yuv starts on
+// 64 x 8 (4 x 1080p 251.7 us, 32 x 8 264.4, 32 x 16 249.5; 640x360 20.3, 21.3, 20.4), the others on
+// 32 x 8 (r3 luma 4 x 1080p 162.0, 64 x 8 167.5, 32 x 16 173.0; r4-yuv 195.9, 205.9, 204.8).  rgb: r2 on
+// 64 x 8 (1280x720 39.8 us, 32 x 8 40.8, 32 x 16 40.6), r3 on 32 x 16 (2 x 1080p 155.4, 64 x 8 157.4, 32 x 8
+// 164.4), r4 on 32 x 8 (231.2, 32 x 16 242.9, 64 x 8 242.7).
 constexpr int ravu_tile_index(int r, int channels, int tile) {
-  if (r != 3 || channels == 0) return tile;
-  if (channels == 2) return tile < 2 ? 1 - tile : tile;
-  return (tile + 2) % 3;
+  const int first = channels == 2 ? (r == 2 ? 2 : r == 3 ? 1 : 0) : (channels == 1 && r == 3 ? 2 : 0);
+  return (tile + first) % 3;
 }
 constexpr int kLiteTileCount = sizeof(kLiteTiles) / sizeof(kLiteTiles[0]);
 constexpr int k3xTileCount = sizeof(k3xTiles) / sizeof(k3xTiles[0]);

@@ -35,44 +35,31 @@ __device__ __forceinline__ void stage_planes(float* tile, const void* base, int 
   h.commit(tile, dt, in_max, in_rmax, W, ox);
 }
 
-// Planes staged per tile: the P input planes, plus for rgb a fourth holding the BT.709
-// luma the hash reads (computed once per staged sample, not once per window use).
+// Floats staged per tile sample: the P input planes and, for rgb, the FP64 BT.709 luma that the
+// hash reads, in the room of two planes behind them (luma_plane).
 template <int CH>
-constexpr int staged_planes() { return CH == 0 ? 1 : (CH == 1 ? 3 : 4); }
+constexpr int staged_planes() { return CH == 0 ? 1 : (CH == 1 ? 3 : 5); }
 
-template <int CH>
-__device__ __forceinline__ float luma_of(const float* t, int o, int n) {
-  return 0.2126f * t[o] + 0.7152f * t[n + o] + 0.0722f * t[2 * n + o];
-}
-
-// rgb: fill plane 3 of a staged tile (n samples per plane) with the luma of planes 0-2;
-// the caller synchronises the block before and after
-template <int CH>
+// rgb: fill the luma of a staged tile (n samples per plane); the caller synchronises the block
+// before and after.
+template <int CH, int NT>
 __device__ __forceinline__ void stage_luma(float* t, int n) {
   if constexpr (CH == 2) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) t[3 * n + i] = luma_of<CH>(t, i, n);
+    fill_luma<NT>(t, reinterpret_cast<double*>(t + 3 * n), n, n);
   }
 }
 
-// Hash-plane value from the staged planes at LDS offset o (plane stride n).
+// The samples that the hash sees of a staged tile (plane stride n), at the offsets of its planes.
 template <int CH>
-__device__ __forceinline__ float luma_f(const float* t, int o, int n) {
-  if (CH == 2) return t[3 * n + o];
-  return t[o];
-}
-template <int CH>
-__device__ __forceinline__ double luma_d(const float* t, int o, int n) {
-#pragma clang fp contract(off)
-  if (CH == 2)
-    return 0.2126 * static_cast<double>(t[o]) + 0.7152 * static_cast<double>(t[n + o]) +
-           0.0722 * static_cast<double>(t[2 * n + o]);
-  return static_cast<double>(t[o]);
+__device__ __forceinline__ const HashSample<CH>* luma_plane(const float* t, int n) {
+  if constexpr (CH == 2) return reinterpret_cast<const double*>(t + 3 * n);
+  else return t;
 }
 
 // Whether full RAVU r2 re-decides a wave's near sites together (wave_tensor), as r3 and r4 do,
-// or each lane its own: together where a sample is the FP64 luma of three (r2 rgb 2 x 1080p
-// 135.5 -> 117.5 us); otherwise its 16 points are soon done, and several of its lanes are near
-// at once (r2 luma together: 99.1 -> 131.9).
+// or each lane its own: its 16 points are soon done, and several of its lanes are near at once
+// (r2 luma together: 99.1 -> 131.9 us); only rgb, whose samples are 8 bytes, is a little faster
+// together (2 x 1080p 129.4, alone 132.0).
 template <int CH>
 constexpr bool wave_redecide() { return CH == 2; }
 
@@ -84,18 +71,19 @@ constexpr bool wave_redecide() { return CH == 2; }
 template <int N, bool FIVE, int RULE, int CH, int PW, int PN>
 __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o) {
   double a, b, d;
-  structure_tensor_fp64<N, FIVE, true>([&](int s) { return luma_d<CH>(t, o + (s % N) * PW + s / N, PN); }, a, b,
-                                          d);
+  const auto l = lds_samples(luma_plane<CH>(t, PN)) + o;
+  structure_tensor_fp64<N, FIVE, true>([&](int s) { return static_cast<double>(l[s % N * PW + s / N]); }, a, b, d);
   return hash_reference<RULE, double>(a, b, d);
 }
 // Hash of this lane's step-1 site; all lanes of the wave together.
 template <int N, int CH, int PW, int PN>
 __device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
-  auto sample = [&](int s) { return luma_f<CH>(t, o + (s % N) * PW + s / N, PN); };
+  const auto* l = luma_plane<CH>(t, PN);
+  auto sample = [&](int s) { return l[o + s % N * PW + s / N]; };
   if constexpr (wave_redecide<CH>()) {
-    return ravu_hash_wave<N, true, RULE_LOG2, wave_sites(CH)>(valid, sample, o, [&](int at) {
-      const float* w = t + at;
-      return [w](int X, int Y) { return luma_d<CH>(w, Y * PW + X, PN); };
+    return ravu_hash_wave<N, true, RULE_LOG2, kWaveSites>(valid, sample, o, [&](int at) {
+      const auto w = lds_samples(l) + at;
+      return [w](int X, int Y) { return static_cast<double>(w[Y * PW + X]); };
     });
   } else {
     float a, b, d;
@@ -124,15 +112,16 @@ __global__ __launch_bounds__(TX * TY) void ravu_3x_kernel(Io io, const __half* _
   stage_planes<P, PH, PW, TX * TY>(tile, in, io.in_dt, io.in_max, io.in_rmax, ft.in_pitch, ft.in_cstride, ft.W, ft.H, x0 - HALO, y0 - HALO);
   __syncthreads();
   if constexpr (CH == 2) {
-    stage_luma<CH>(tile, PN);
+    stage_luma<CH, TX * TY>(tile, PN);
     __syncthreads();
   }
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
   const int x = x0 + tx, y = y0 + ty;
   if (x >= ft.W || y >= ft.H) return;
   auto off = [&](int i) { return (ty + i % N) * PW + tx + i / N; };  // sample i = X*N + Y
-  const Bucket bk = ravu_hash<N, false, RULE_3X>([&](int i) { return luma_f<CH>(tile, off(i), PN); },
-                                                 [&](int i) { return luma_d<CH>(tile, off(i), PN); });
+  const auto* lum = luma_plane<CH>(tile, PN);
+  const Bucket bk = ravu_hash<N, false, RULE_3X>([&](int i) { return lum[off(i)]; },
+                                                 [&](int i) { return static_cast<double>(lum[off(i)]); });
   const int row = bucket_row<RULE_3X>(bk, 216);
   if (io.buckets) io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y) * ft.W + x] = row;
   const __half* lrow = lut + static_cast<int64_t>(row) * NTEX * 4;
@@ -285,7 +274,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(6))) vo
                   y0 - (R - 1));
   __syncthreads();
   if constexpr (CH == 2) {
-    stage_luma<CH>(tile, PN);
+    stage_luma<CH, TX * TY>(tile, PN);
     __syncthreads();
   }
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
@@ -313,19 +302,19 @@ __device__ __host__ constexpr int lat2x(int X, int Y) { return STEP == 2 ? X + Y
 template <int N, int STEP>
 __device__ __host__ constexpr int lat2y(int X, int Y) { return STEP == 2 ? Y - X : Y - X + 1; }
 
-// FP64 samples of a step 2 / 3 window, `at` = LDS offset of the site in the staged input (px and
+// FP64 samples of a step 2 / 3 window, `at` = offset of the site in the staged input (px and
 // py have the same parity; the int11 tile follows the input's).  It keeps the window's lowest
 // address, so the reads' offsets are non-negative immediates (otherwise the addresses are
 // registers of their own).
-template <int N, int STEP, int CH, int PW, int PN>
+// (`lum`: the samples that the hash sees of the input; int11's are NEXT further.)
+template <int N, int STEP, int PW, int NEXT, typename T>
 struct LatticeWindow {
   static constexpr int LOW = N / 2 * (PW + 1);
-  typename TilePointer<CH>::T t;
-  __device__ __forceinline__ LatticeWindow(const float* hk, int at)
-      : t((typename TilePointer<CH>::T)(hk + at - LOW)) {}
+  LdsSamples<T> t;
+  __device__ __forceinline__ LatticeWindow(const T* lum, int at) : t(lds_samples(lum) + at - LOW) {}
   __device__ __forceinline__ double operator()(int X, int Y) const {
     const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
-    return luma_d<CH>((const float*)t, LOW + (py >> 1) * PW + (px >> 1) + (px & 1) * (staged_planes<CH>() * PN), PN);
+    return t[LOW + (py >> 1) * PW + (px >> 1) + (px & 1) * NEXT];
   }
 };
 
@@ -344,14 +333,19 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
     const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
     return (px & 1) ? i11 + base + ((py - 1) >> 1) * PW + ((px - 1) >> 1) : hk + base + (py >> 1) * PW + (px >> 1);
   };
-  auto sample = [&](int i) { return luma_f<CH>(src(i), 0, PN); };
+  auto sample = [&](int i) {
+    const int px = lat2x<N, STEP>(i / N, i % N), py = lat2y<N, STEP>(i / N, i % N);
+    return (px & 1) ? luma_plane<CH>(i11, PN)[base + ((py - 1) >> 1) * PW + ((px - 1) >> 1)]
+                    : luma_plane<CH>(hk, PN)[base + (py >> 1) * PW + (px >> 1)];
+  };
   Bucket bk;
   if constexpr (wave_redecide<CH>()) {
-    bk = ravu_hash_wave<N, true, RULE_LOG2, wave_sites(CH)>(valid, sample, base, [&](int o) {
-      return LatticeWindow<N, STEP, CH, PW, PN>(hk, o);
+    bk = ravu_hash_wave<N, true, RULE_LOG2, kWaveSites>(valid, sample, base, [&](int o) {
+      constexpr int NEXT = staged_planes<CH>() * PN * static_cast<int>(sizeof(float)) / static_cast<int>(sizeof(HashSample<CH>));
+      return LatticeWindow<N, STEP, PW, NEXT, HashSample<CH>>(luma_plane<CH>(hk, PN), o);
     });
   } else {
-    bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return luma_d<CH>(src(i), 0, PN); });
+    bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return static_cast<double>(sample(i)); });
   }
   if (!valid) return;
   const int row = bucket_row<RULE_LOG2>(bk, 648);
@@ -400,8 +394,8 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_kernel(Io io, const __ha
   }
   __syncthreads();
   if constexpr (CH == 2) {
-    stage_luma<CH>(hk, PN);
-    stage_luma<CH>(i11, PN);
+    stage_luma<CH, TX * TY>(hk, PN);
+    stage_luma<CH, TX * TY>(i11, PN);
     __syncthreads();
   }
   const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
@@ -459,11 +453,11 @@ struct SepTensor {
     for (int k = 0; k < RUN; ++k) out[k] = {{0.f, 0.f}, {0.f, 0.f}, 0.f};
 #pragma unroll
     for (int r = 0; r < M + RUN - 1; ++r) {
-      const float xc = s(1, r) - s(-1, r);
-      const float xf = fmaf(8.0f, xc, s(-2, r) - s(2, r));
-      const float yc = s(0, r + 1) - s(0, r - 1);
+      const float xc = difference(s(1, r), s(-1, r));
+      const float xf = fmaf(8.0f, xc, difference(s(-2, r), s(2, r)));
+      const float yc = difference(s(0, r + 1), s(0, r - 1));
       float yf = 0.f;
-      if (uses<RUN>(true, r)) yf = fmaf(8.0f, yc, s(0, r - 2) - s(0, r + 2));
+      if (uses<RUN>(true, r)) yf = fmaf(8.0f, yc, difference(s(0, r - 2), s(0, r + 2)));
       const float xc2 = xc * xc, xf2 = xf * xf;
       const float cc = xc * yc, fc = xf * yc, yc2 = yc * yc;
       const float cf = xc * yf, ff = xf * yf, yf2 = yf * yf;
@@ -495,6 +489,18 @@ struct SepTensor {
   }
 };
 
+// Floats of the tables' LDS (tn entries of five).  rgb: the FP64 lumas (n of them) from which the sums
+// are taken live there first, the tables then take their place, and a block with near sites
+// fills them in again for the re-decision.  With both kept at once r3-rgb's kernels had 16 waves
+// per compute unit instead of 24.
+template <int CH>
+constexpr int table_floats(int tn, int n) { return CH == 2 && 2 * n > 5 * tn ? 2 * n : 5 * tn; }
+template <int CH>
+__device__ __forceinline__ const HashSample<CH>* hash_samples(const float* tile, const float* tab) {
+  if constexpr (CH == 2) return reinterpret_cast<const double*>(tab);
+  else return tile;
+}
+
 // Weight p (texel p / 4, component p % 4) of a LUT row held raw.
 template <int NTEX>
 struct RawRow {
@@ -523,32 +529,39 @@ __global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))
   constexpr int PW = staged_width(TX + N - 1), PH = TY + N - 1, PN = PW * PH;
   using Sep = SepTensor<N>;
   constexpr int RUN = 4, NC = TX + Sep::M - 1;  // table columns: staged columns 1 .. NC
-  static_assert(TY % RUN == 0, "whole runs");
-  __shared__ __attribute__((aligned(16))) float tile[staged_planes<CH>() * PN];
-  __shared__ float2 tc[NC * TY], tf[NC * TY];
-  __shared__ float td[NC * TY];
+  constexpr int RUNS = NC * (TY / RUN), TN = NC * TY;
+  static_assert(TY % RUN == 0 && RUNS <= NT, "whole runs, one per thread");
+  __shared__ __attribute__((aligned(16))) float tile[P * PN];
+  __shared__ __attribute__((aligned(16))) float tab[table_floats<CH>(TN, PN)];
+  float2 *tc = reinterpret_cast<float2*>(tab), *tf = tc + TN;
+  float* td = reinterpret_cast<float*>(tf + TN);
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
   stage_planes<P, PH, PW, NT>(tile, frame_in(io, f), io.in_dt, io.in_max, io.in_rmax, ft.in_pitch, ft.in_cstride,
                               ft.W, ft.H, x0 - (R - 1), y0 - (R - 1));
   __syncthreads();
+  const HashSample<CH>* lum = hash_samples<CH>(tile, tab);
   if constexpr (CH == 2) {
-    stage_luma<CH>(tile, PN);
+    fill_luma<NT>(tile, reinterpret_cast<double*>(tab), PN, PN);
     __syncthreads();
   }
-  const float* lum = tile + (CH == 2 ? 3 * PN : 0);
-  for (int i = threadIdx.x; i < NC * (TY / RUN); i += NT) {
-    const int q = i / NC, c = i - q * NC;
-    const float* p = lum + (q * RUN + 1) * PW + c + 1;
+  {
+    const int i = threadIdx.x, q = i / NC, c = i - q * NC;
     typename Sep::Column v[RUN];
-    Sep::template columns<RUN>([&](int dx, int dy) { return p[dy * PW + dx]; }, v);
+    if (i < RUNS) {
+      const auto* p = lum + (q * RUN + 1) * PW + c + 1;
+      Sep::template columns<RUN>([&](int dx, int dy) { return p[dy * PW + dx]; }, v);
+    }
+    if constexpr (CH == 2) __syncthreads();  // the tables take the lumas' place
+    if (i < RUNS) {
 #pragma unroll
-    for (int k = 0; k < RUN; ++k) {
-      const int e = (q * RUN + k) * NC + c;
-      tc[e] = v[k].c;
-      tf[e] = v[k].f;
-      td[e] = v[k].d;
+      for (int k = 0; k < RUN; ++k) {
+        const int e = (q * RUN + k) * NC + c;
+        tc[e] = v[k].c;
+        tf[e] = v[k].f;
+        td[e] = v[k].d;
+      }
     }
   }
   __syncthreads();
@@ -557,21 +570,45 @@ __global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))
   const bool valid = x < ft.W && y < ft.H, second = y + 1 < ft.H;
   const int o = ty * PW + tx;
   int row[2] = {0, 0};
+  bool near[2];
+  auto decide = [&](int s, Bucket& bk) {
+    redecide<N, true, RULE_LOG2, kWaveSites>(near[s], o, [&](int at) {
+      const auto w = lds_samples(lum) + at + s * PW;
+      return [w](int X, int Y) { return static_cast<double>(w[Y * PW + X]); };
+    }, bk);
+    if (CH != 2 || near[s]) row[s] = bucket_row<RULE_LOG2>(bk, 648);
+  };
+  auto report = [&](int s) {
+    if (io.buckets && valid && (s == 0 || second))
+      io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y + s) * ft.W + x] = row[s];
+  };
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const int e = (ty + s) * NC + tx;
     float a, b, d;
     Sep::site([&](bool five, int i) { return five ? tf[e + i] : tc[e + i]; }, [&](int i) { return td[e + i]; }, a, b, d);
-    bool near = false;
-    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
-    redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid && (s == 0 || second), o, [&](int at) {
-      const auto w = (typename TilePointer<CH>::T)(tile + at + s * PW);
-      return [w](int X, int Y) { return luma_d<CH>((const float*)w, Y * PW + X, PN); };
-    }, bk);
-    row[s] = bucket_row<RULE_LOG2>(bk, 648);
-    if (io.buckets && valid && (s == 0 || second))
-      io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y + s) * ft.W + x] = row[s];
+    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near[s]);
+    near[s] = near[s] && valid && (s == 0 || second);
+    if constexpr (CH == 2) {
+      row[s] = bucket_row<RULE_LOG2>(bk, 648);
+    } else {
+      decide(s, bk);
+      report(s);
+    }
     __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (CH == 2) {
+    if (__syncthreads_or(near[0] || near[1])) {
+      fill_luma<NT>(tile, reinterpret_cast<double*>(tab), PN, PN);
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        Bucket bk{};
+        decide(s, bk);
+      }
+    }
+    report(0);
+    report(1);
   }
   if (!valid) return;
   constexpr int NTEX = RavuLut<N>::NTEX;
@@ -623,10 +660,11 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
   constexpr int H = Sep::M / 2;
   // tables by int11 site (-H .. TX - 1, -H .. TY - 1) and input pixel (1-H .. TX - 1, 1-H .. TY - 1)
   constexpr int NC = TX + H, NR = TY + H, EC = NC - 1, ER = NR - 1, EN = EC * ER, TN = EN + NC * NR;
-  __shared__ __attribute__((aligned(16))) float tiles[2][staged_planes<CH>() * PN];
+  __shared__ __attribute__((aligned(16))) float tiles[2][P * PN];
   float *hk = tiles[0], *i11 = tiles[1];  // input (HOOKED), ravu_int11
-  __shared__ float2 tc[TN], tf[TN];  // input pixels' entries, then int11 sites'
-  __shared__ float td[TN];
+  __shared__ __attribute__((aligned(16))) float tab[table_floats<CH>(TN, 2 * PN)];
+  float2 *tc = reinterpret_cast<float2*>(tab), *tf = tc + TN;  // input pixels' entries, then int11 sites'
+  float* td = reinterpret_cast<float*>(tf + TN);
   const FrameTile ft = frame_tile<TX, TY>(io, blockIdx.x, total);
   const int f = ft.f;
   const int x0 = ft.x0, y0 = ft.y0;
@@ -641,33 +679,59 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
     b.commit(i11, DT_F32, 1.f, 1.f, ft.W, x0 - R);
   }
   __syncthreads();
+  // the samples that the hash sees: the input's, then (NEXT further) int11's
+  constexpr int NEXT = CH == 2 ? PN : P * PN;
+  const HashSample<CH>* lum = hash_samples<CH>(hk, tab);
+  auto lumas = [&] {
+    fill_luma<NT>(hk, reinterpret_cast<double*>(tab), PN, PN);
+    fill_luma<NT>(i11, reinterpret_cast<double*>(tab) + PN, PN, PN);
+  };
   if constexpr (CH == 2) {
-    stage_luma<CH>(hk, PN);
-    stage_luma<CH>(i11, PN);
+    lumas();
     __syncthreads();
   }
   {
-    const float* lh = hk + (CH == 2 ? 3 * PN : 0);
-    const float* li = i11 + (CH == 2 ? 3 * PN : 0);
-    for (int i = threadIdx.x; i < NC * NR; i += NT) {
+    constexpr int E = (NC * NR + NT - 1) / NT;
+    typename Sep::Column v[CH == 2 ? E : 1][2];
+    auto sums = [&](int i, typename Sep::Column (&out)[2]) {
       const int q = i / NC, c = i - q * NC;
-      const int o = (q - H + R) * PW + c - H + R;  // input pixel (c - H, q - H)
-      typename Sep::Column v[2];
+      const auto* p = lum + (q - H + R) * PW + c - H + R;  // input pixel (c - H, q - H)
       Sep::template columns<2>(
           [&](int dx, int dy) {  // lattice steps from that pixel
             const int u = dx + dy, w = dy - dx;
-            return (u & 1) ? li[o + ((w - 1) >> 1) * PW + ((u - 1) >> 1)] : lh[o + (w >> 1) * PW + (u >> 1)];
+            return p[(u & 1) ? NEXT + ((w - 1) >> 1) * PW + ((u - 1) >> 1) : (w >> 1) * PW + (u >> 1)];
           },
-          v);
+          out);
+    };
+    auto put = [&](int i, const typename Sep::Column (&in)[2]) {
+      const int q = i / NC, c = i - q * NC;
       if (q > 0 && c > 0) {
         const int e = (q - 1) * EC + c - 1;
-        tc[e] = v[0].c;
-        tf[e] = v[0].f;
-        td[e] = v[0].d;
+        tc[e] = in[0].c;
+        tf[e] = in[0].f;
+        td[e] = in[0].d;
       }
-      tc[EN + i] = v[1].c;
-      tf[EN + i] = v[1].f;
-      td[EN + i] = v[1].d;
+      tc[EN + i] = in[1].c;
+      tf[EN + i] = in[1].f;
+      td[EN + i] = in[1].d;
+    };
+    if constexpr (CH == 2) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = static_cast<int>(threadIdx.x) + e * NT;
+        if (i < NC * NR) sums(i, v[e]);
+      }
+      __syncthreads();  // the tables take the lumas' place
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = static_cast<int>(threadIdx.x) + e * NT;
+        if (i < NC * NR) put(i, v[e]);
+      }
+    } else {
+      for (int i = threadIdx.x; i < NC * NR; i += NT) {
+        sums(i, v[0]);
+        put(i, v[0]);
+      }
     }
   }
   __syncthreads();
@@ -686,6 +750,20 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
     return (px & 1) ? i11 + base + ((py - 1) >> 1) * PW + ((px - 1) >> 1) : hk + base + (py >> 1) * PW + (px >> 1);
   };
   int row[2];
+  bool near[2];
+  auto decide = [&](int s, Bucket& bk) {
+    if (s == 0)
+      redecide<N, true, RULE_LOG2, kWaveSites>(
+          near[s], base, [&](int o) { return LatticeWindow<N, 2, PW, NEXT, HashSample<CH>>(lum, o); }, bk);
+    else
+      redecide<N, true, RULE_LOG2, kWaveSites>(
+          near[s], base, [&](int o) { return LatticeWindow<N, 3, PW, NEXT, HashSample<CH>>(lum, o); }, bk);
+    if (CH != 2 || near[s]) row[s] = bucket_row<RULE_LOG2>(bk, 648);
+  };
+  auto report = [&](int s) {
+    if (io.buckets && valid)
+      io.buckets[f * io.bucket_bstride + (s + 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row[s];
+  };
 #pragma unroll
   for (int s = 0; s < 2; ++s) {  // step 2, step 3: grid index i is column i + 1, i
     float a, b, d;
@@ -693,18 +771,28 @@ __global__ __launch_bounds__(TX * TY) void ravu_lattice_pair_kernel(Io io, const
           return five ? tf[entry(i + 1 - s)] : tc[entry(i + 1 - s)];
         },
         [&](int i) { return td[entry(i + 1 - s)]; }, a, b, d);
-    bool near = false;
-    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near);
-    if (s == 0)
-      redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
-                                   [&](int o) { return LatticeWindow<N, 2, CH, PW, PN>(hk, o); }, bk);
-    else
-      redecide<N, true, RULE_LOG2, wave_sites(CH)>(near && valid, base,
-                                   [&](int o) { return LatticeWindow<N, 3, CH, PW, PN>(hk, o); }, bk);
-    row[s] = bucket_row<RULE_LOG2>(bk, 648);
-    if (io.buckets && valid)
-      io.buckets[f * io.bucket_bstride + (s + 1) * plane + static_cast<int64_t>(y) * ft.W + x] = row[s];
+    Bucket bk = hash_fast<RULE_LOG2>(a, b, d, &near[s]);
+    near[s] = near[s] && valid;
+    if constexpr (CH == 2) {
+      row[s] = bucket_row<RULE_LOG2>(bk, 648);
+    } else {
+      decide(s, bk);
+      report(s);
+    }
     __builtin_amdgcn_sched_barrier(0);  // one step's registers live at a time
+  }
+  if constexpr (CH == 2) {
+    if (__syncthreads_or(near[0] || near[1])) {
+      lumas();
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        Bucket bk{};
+        decide(s, bk);
+      }
+    }
+    report(0);
+    report(1);
   }
   if (!valid) return;
   constexpr int NTEX = RavuLut<N>::NTEX;

@@ -99,20 +99,6 @@ struct PhaseFetch {
   }
 };
 
-template <int CH>
-__device__ __forceinline__ float zluma_f(const float* t, int o, int n) {
-  if (CH == 2) return 0.2126f * t[o] + 0.7152f * t[n + o] + 0.0722f * t[2 * n + o];
-  return t[o];
-}
-template <int CH>
-__device__ __forceinline__ double zluma_d(const float* t, int o, int n) {
-#pragma clang fp contract(off)
-  if (CH == 2)
-    return 0.2126 * static_cast<double>(t[o]) + 0.7152 * static_cast<double>(t[n + o]) +
-           0.0722 * static_cast<double>(t[2 * n + o]);
-  return static_cast<double>(t[o]);
-}
-
 // Stage the part of the PH x PW staging area that a tile's outputs read: the uh x uw
 // samples per plane around its base pixels (at 2x 8 x 20 of 12 x 36), clamp-to-edge, at
 // the area's row stride PW.  AR forms store each sample's anti-ringing powers beside it
@@ -233,24 +219,36 @@ __device__ __forceinline__ float zoom_ring(float v, float hi, float lo, float hi
   return v * (1.0f - 0.8f) + cl * 0.8f;
 }
 
+// The samples that the hash sees of a staged tile (n per plane): for rgb the FP64 luma, filled into
+// `luma` here for `count` samples; the caller synchronises the block before and after.
+template <int CH, int NT>
+__device__ __forceinline__ const HashSample<CH>* zoom_luma(const float* tile, double* luma, int n, int count) {
+  if constexpr (CH == 2) {
+    fill_luma<NT>(tile, luma, n, count);
+    return luma;
+  } else {
+    return tile;
+  }
+}
+
 // Hash every base pixel of a tile (nbx x nby) into bucket[by * BX + bx]: the unclamped LUT row
 // (bucket 9-row blocks are clamped per texel by the bilinear fetch, as the sampler does).
 // r2's near lanes evaluate their own windows (16 points: a turn of the wave is no cheaper, and the
 // kernel is smaller: zoom-ar-r2-rgb 4 x 720p -> 1440p 210 -> 204 us, ar-r2 134 -> 127).  TAB only
 // tells the kernels apart: the out-of-line evaluation follows its caller's register budget.
-template <int R, bool AR, int CH, bool TAB, int BX, int PW, int PN, int NT>
-__device__ __forceinline__ void hash_bases(const float* tile, int* bucket, int nbx, int nby) {
+template <int R, bool AR, int CH, bool TAB, int BX, int PW, int NT>
+__device__ __forceinline__ void hash_bases(const HashSample<CH>* lum, int* bucket, int nbx, int nby) {
   constexpr int N = 2 * R;
   // (whole waves: the re-decision takes all lanes; those past the last base pixel repeat it)
   for (int i0 = threadIdx.x & ~63; i0 < nbx * nby; i0 += NT) {
     const int lane_i = i0 + static_cast<int>(threadIdx.x & 63), i = min(lane_i, nbx * nby - 1);
     const int by = i / nbx, bx = i - by * nbx;
     auto off = [&](int s) { return (by + s % N) * PW + bx + s / N; };
-    auto sample = [&](int s) { return zluma_f<CH>(tile, off(s), PN); };
-    const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, R == 2 ? 0 : wave_sites(CH)>(
+    auto sample = [&](int s) { return lum[off(s)]; };
+    const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, R == 2 ? 0 : kWaveSites>(
         lane_i == i, sample, by * PW + bx, [&](int o) {
-          const auto t = (typename TilePointer<CH>::T)(tile + o);
-          return [t](int X, int Y) { return zluma_d<CH>((const float*)t, Y * PW + X, PN); };
+          const auto t = lds_samples(lum) + o;
+          return [t](int X, int Y) { return static_cast<double>(t[Y * PW + X]); };
         });
     if (lane_i == i) bucket[by * BX + bx] = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
   }
@@ -273,7 +271,9 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   constexpr int ROWS = 2592;             // 288 buckets x 9 phases
   constexpr int BX = TX + 1, BY = TY + 1;  // base pixels a tile can touch (ratio in/out < 1)
   constexpr int PW = BX + N - 1, PH = BY + N - 1, PN = PW * PH;
-  __shared__ float tile[P * PN];
+  __shared__ __attribute__((aligned(16))) float tile[P * PN];
+  static_assert(PN % 2 == 0, "lumas in pairs");
+  __shared__ __attribute__((aligned(16))) double luma[CH == 2 ? PN : 1];
   __shared__ int bucket[BY * BX];
   // AR: per staged sample (l + 0.1)^32, (1.1 - l)^32 and the ^33 terms, computed once per
   // sample instead of once per output pixel that reads it (about 25 at 2x)
@@ -292,7 +292,9 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   stage_used<P, PH, PW, TX * TY, AR>(tile, pw, in, io.in_dt, io.in_max, io.in_rmax, io.in_pitch, io.in_cstride, io.W, io.H,
                             bx0 - (R - 1), by0 - (R - 1), nbx + N - 1, nby + N - 1);
   __syncthreads();
-  hash_bases<R, AR, CH, TAB, BX, PW, PN, TX * TY>(tile, bucket, nbx, nby);
+  const auto* lum = zoom_luma<CH, TX * TY>(tile, luma, PN, (nby + N - 1) * PW);
+  if constexpr (CH == 2) __syncthreads();
+  hash_bases<R, AR, CH, TAB, BX, PW, TX * TY>(lum, bucket, nbx, nby);
   __syncthreads();
 
   const int ox = ox0 + threadIdx.x % TX, oy = oy0 + threadIdx.x / TX;
@@ -426,7 +428,9 @@ __global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const fl
   constexpr int BX = TX, BY = TY + 1;
   constexpr int PW = BX + N - 1, PH = BY + N - 1, PN = PW * PH;
   constexpr int NT = AR ? 4 : 2;
-  __shared__ float tile[P * PN];
+  __shared__ __attribute__((aligned(16))) float tile[P * PN];
+  static_assert(PN % 2 == 0, "lumas in pairs");
+  __shared__ __attribute__((aligned(16))) double luma[CH == 2 ? PN : 1];
   __shared__ int bucket[BY * BX];
   __shared__ float4 pw[AR ? P * PN : 1];
 
@@ -441,7 +445,9 @@ __global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const fl
                                      io.in_cstride, io.W, io.H, bx0 - (R - 1), by0 - (R - 1), nbx + N - 1,
                                      nby + N - 1);
   __syncthreads();
-  hash_bases<R, AR, CH, true, BX, PW, PN, TX * TY>(tile, bucket, nbx, nby);
+  const auto* lum = zoom_luma<CH, TX * TY>(tile, luma, PN, (nby + N - 1) * PW);
+  if constexpr (CH == 2) __syncthreads();
+  hash_bases<R, AR, CH, true, BX, PW, TX * TY>(lum, bucket, nbx, nby);
   __syncthreads();
 
   const int lbx = threadIdx.x % TX, oy = oy0 + threadIdx.x / TX;
