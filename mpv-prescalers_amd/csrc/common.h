@@ -450,11 +450,12 @@ __device__ __forceinline__ void structure_tensor(Get get, float& a, float& b, fl
   a = b = d = 0.f;
 #pragma unroll
   for (int X = GG::P0; X < GG::P1; ++X) {
-    // (FP64 samples: the columns that three derivatives need live at a time)
+    // FP64 samples: one column of points at a time (7 x 7 windows one point: 100 -> 62 VGPRs, and
+    // 3x-r4-rgb 1280x720 48.6 -> 47.4 us; at 6 x 6 that took zoom-r3-rgb at 1.25x from 29.5 to 34.1)
     if constexpr (sizeof(get(0)) == 8) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int Y = GG::P0; Y < GG::P1; ++Y) {
-      if constexpr (sizeof(get(0)) == 8) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (sizeof(get(0)) == 8 && N == 7) __builtin_amdgcn_sched_barrier(0);
       const float gx = deriv_unscaled<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
       const float gy = deriv_unscaled<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
       const double cx = deriv_scale<N, FIVE>(X), cy = deriv_scale<N, FIVE>(Y);
