@@ -171,6 +171,19 @@ __device__ __forceinline__ void stage_used(float* tile, float4* pw, const void* 
 // bucket 288 (the texel rows clamp), so rows -1..288 cover every bucket value.
 constexpr int kZoomRowLo = -1, kZoomRows = 290;
 constexpr int kZoomMaxPhasePairs = 64;
+// float4s from one bucket row's entries to the next.  L1 serves 16 bytes per lane, four lanes per
+// cycle, if the four lie in different 16-byte columns of their 64-byte halves of lines.  A lane reads
+// its own row's entries at an offset that all lanes share, so with rows a multiple of 64 bytes apart
+// every lane wants the same column.  An odd stride puts neighbouring rows into different ones.
+// Where neighbouring lanes' column phases already differ in it (three or more phases, 160 bytes
+// apart) the stride stays.  Measured at 2x, where noisy frames were bound by this path (texture data busy
+// for the whole launch, 49 cycles per load): r3 4 x 720p noise 226 -> 159 us, video 113 -> 91; r3-yuv
+// 235 -> 175, 129 -> 120; ar-r2 195 -> 140, 114 -> 94; r2 103 -> 77, 75 -> 71; at 1.5x ar-r2 720p 37.0 ->
+// 28.9, 34.4 -> 29.8.  (r3 at 1.25x with an odd stride: 28.1 -> 30.1.)
+__device__ __host__ constexpr int zoom_row_stride(int nphx, int nphy, int groups, int nt) {
+  const int n = nphx * nphy * groups * nt;
+  return nphx == 2 || groups * nt % 4 == 0 ? n | 1 : n;
+}
 
 template <int R, bool AR>
 __global__ __launch_bounds__(256) void zoom_table_kernel(const __half* __restrict__ lut,
@@ -191,7 +204,7 @@ __global__ __launch_bounds__(256) void zoom_table_kernel(const __half* __restric
   const Phase phx = phase_of(px, in_w, out_w), phy = phase_of(py, in_h, out_h);
   const float txf = 8.f * phx.f, txi = 8.f * (1.f - phx.f);
   const float tyf = 8.f * phy.f, tyi = 8.f * (1.f - phy.f);
-  float4* e = wtab + static_cast<int64_t>(i) * NT;
+  float4* e = wtab + (row - kZoomRowLo) * zoom_row_stride(nphx, nphy, GROUPS, NT) + ((py * nphx + px) * GROUPS + g) * NT;
   e[0] = PhaseFetch<GROUPS>(lut, ROWS, txf, row, tyf).get(g);
   e[1] = PhaseFetch<GROUPS>(lut, ROWS, txi, row, tyi).get(g);
   if (AR) {
@@ -312,7 +325,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
   const float4* wt = nullptr;
   if constexpr (TAB) {
     const int trow = min(max(row, kZoomRowLo), kZoomRowLo + kZoomRows - 1) - kZoomRowLo;
-    wt = wtab + static_cast<int64_t>(((trow * nphy + phy.z) * nphx + phx.z) * GROUPS) * NT;
+    wt = wtab + trow * zoom_row_stride(nphx, nphy, GROUPS, NT) + (phy.z * nphx + phx.z) * (GROUPS * NT);
   }
   float res[P], hi[P], lo[P], hi2[P], lo2[P];
 #pragma unroll
@@ -464,7 +477,7 @@ __global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const fl
   }
   const int trow = min(max(row, kZoomRowLo), kZoomRowLo + kZoomRows - 1) - kZoomRowLo;
   const float4* wt[2];
-  wt[1] = wtab + static_cast<int64_t>((trow * nphy + phy.z) * 2) * (GROUPS * NT);
+  wt[1] = wtab + trow * zoom_row_stride(2, nphy, GROUPS, NT) + phy.z * (2 * GROUPS * NT);
   wt[0] = wt[1] + GROUPS * NT;
   const float* tp = tile + lby * PW + lbx;
   const float4* pp = pw + lby * PW + lbx;
@@ -605,7 +618,7 @@ int zoom_plan_create(mpx_ctx* ctx, mpx_plan* plan, int in_w, int in_h, int out_w
   const bool ar = plan->v->ar != 0;
   const int groups = (2 * r * 2 * r / 2 + 3) / 4;
   const int entries = kZoomRows * nphy * nphx * groups;
-  const size_t bytes = static_cast<size_t>(entries) * (ar ? 4 : 2) * sizeof(float4);
+  const size_t bytes = static_cast<size_t>(kZoomRows) * zoom_row_stride(nphx, nphy, groups, ar ? 4 : 2) * sizeof(float4);
   void* p = nullptr;
   if (ctx->alloc(bytes, &p)) return MPX_OK;  // over the budget: per-pixel interpolation
   mpx_host::DeviceScope ds;
