@@ -562,15 +562,20 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 // in FP32).  Sets *near, and the caller re-decides in FP64, when a decision may differ from
 // the exact one.  The tensor's own FP32 error (u = 2^-24): differences of exact samples are off by
 // u each, which the five-point stencil can amplify by cancellation, but never past 1.83 u of the
-// tensor's norm (the largest ratio over all 8 x 8 windows, an eigenvalue; 6 x 6: 1.69, central
-// and border stencils: 1); with the derivative's own rounding that is 6 u of a, d.  36 terms,
-// each squared and weighted, summed one after the other then give a, d within 44 u of themselves
-// and b within 44 u T / 2 (column sums, SepTensor: two levels of at most six terms and rounded
-// 1-D weights, 22 u), hence sqrt(L1) within a relative 44 u = 2.6e-6 (margin 3.8e-6), L2 within
-// 44 u T (6.9e-6 T = 115 u), mu within 59 u at 1/4 and 99 u at 1/2 (6e-6 = 100 u), and the angle
-// within 31 u T / (2 delta) (32 u, plus 1e-5 units for the evaluation, whose error is below
+// tensor's norm (the largest ratio over all 8 x 8 windows, an eigenvalue; 6 x 6: 1.69, central and
+// border stencils: 1); the five-point form adds a rounding of its own.  Both count twice in a
+// square, beside one rounding each of the product and the weight and one per term of a running
+// sum.  That puts a and d within K u of themselves and b within K u T / 2, K = 13 for 5 x 5 windows
+// (9 terms), 29 for 7 x 7 (25), 20 for 4 x 4 (16; 31 for rgb, rounded relative to an inner sample), 24
+// for 6 x 6 (16), 17 and 21 for the column sums of 6 x 6 and 8 x 8 (SepTensor: two levels of four or six
+// terms).  With K <= 31, sqrt(L1) lies within a relative 31 u = 1.9e-6 (margin 3.8e-6), b within
+// 15.5 u T (16 u), L2 within 31 u T (99 u), mu within 42 u at 1/4 and 70 u at 1/2 (6e-6 = 100 u), the
+// angle within 22 u T / (2 delta) (32 u, plus 1e-5 units for the evaluation, whose error is below
 // 5e-6).  A sample that is itself rounded, like an rgb luma in FP32, has no place in this bound:
 // see HashSample.  Exact cases (flat window T = 0, b = 0 exactly) are never near.
+// The margin of b decides which frames of thin horizontal and vertical lines are near everywhere:
+// with 24 u, a line grid 1280x720 took lite-r3 18.9 us instead of 15.7, r3 80.1 instead of 73.9,
+// r4-rgb (of an FP32 luma) 339 instead of 154, zoom-r3 at 1.5x 44.0 instead of 36.6.
 // Bound by VALU issue: the exactly rounded sqrtf, the library atan2f and log2f that this
 // replaces took about 75 of a hash's ~150 instructions, and an angle margin of 2.4e-4 units
 // sent 3-4x as many sites to FP64.  Measured: ravu-r3 1366x768 44.3 -> 37.5 us, r4-yuv
@@ -579,7 +584,7 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 template <int RULE>
 __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* near) {
   const float eps = 1.192092896e-7f;
-  const float rel = 4e-6f, u24 = 24.0f * 5.9604645e-8f;
+  const float rel = 4e-6f, u16 = 16.0f * 5.9604645e-8f;
   const float T = a + d;
   const float h = (a - d) * 0.5f;
   const float delta = __builtin_amdgcn_sqrtf(fmaf(h, h, b * b));
@@ -611,8 +616,8 @@ __device__ __forceinline__ Bucket hash_fast(float a, float b, float d, bool* nea
   Bucket bk;
   bk.angle = static_cast<int>(floorf(u));
   bk.coherence = mu >= 0.5f ? 2 : (mu >= 0.25f ? 1 : 0);
-  bool n = fabsf(ab - eps) <= fmaf(u24, T, rel * eps);
-  n |= fabsf(L2) <= (rel + 2.0f * u24) * T && !(b == 0.f && fminf(a, d) == 0.f);
+  bool n = fabsf(ab - eps) <= fmaf(u16, T, rel * eps);
+  n |= fabsf(L2) <= (rel + 2.0f * u16) * T && !(b == 0.f && fminf(a, d) == 0.f);
   const float cond = (24.0f / kPiF) * 32.0f * 5.9604645e-8f * T * __builtin_amdgcn_rcpf(fmaxf(2.0f * delta, 1e-30f));
   n |= !bsmall && fabsf(u - rintf(u)) <= 1e-5f + cond;
   if (RULE == RULE_LOG2) {
