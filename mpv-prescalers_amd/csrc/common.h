@@ -468,31 +468,35 @@ __device__ __forceinline__ void structure_tensor(Get get, float& a, float& b, fl
   }
 }
 
-// The same in FP64, in the reference's rounding steps and order, by one lane.  LEAN (large
-// windows): one derivative at a time (scheduling barriers, the partial sums pinned), so the
-// rare re-decision does not hold the window in FP64 registers and set every wave's occupancy.
+// The same in FP64, in the reference's rounding steps and order, by one lane; get(i) returns the
+// sample as it is stored.  LEAN (large windows): a column of points at a time, or one point for 8 x 8
+// windows and FP64 samples (scheduling barriers, the partial sums pinned), so the rare re-decision
+// does not hold the window in FP64 registers and set every wave's occupancy.
+// Bound by the latency of its LDS reads: with one derivative at a time large flat shapes 1280x720 took
+// r3 46.3 us, now 44.0, r3-yuv 58.9 -> 55.7, r4-yuv line grid 148 -> 137.  (r4 by columns: 38.2 -> 39.1 on
+// ordinary frames, five waves per SIMD instead of six; zoom-r3-rgb at 1.5x 36.4 -> 37.4.)
 template <int N, bool FIVE, bool LEAN, typename Get>
 __device__ __forceinline__ void structure_tensor_fp64(Get get, double& a, double& b, double& d) {
 #pragma clang fp contract(off)
   using GG = GradGrid<N>;
+  constexpr bool POINTS = N == 8 || sizeof(get(0)) == 8;
+  auto sample = [&](int i) { return static_cast<double>(get(i)); };
   a = b = d = 0.0;
 #pragma unroll
   for (int X = GG::P0; X < GG::P1; ++X) {
 #pragma unroll
     for (int Y = GG::P0; Y < GG::P1; ++Y) {
-      double gx = deriv<N, FIVE>([&](int k) { return get(k * N + Y); }, X);
-      if constexpr (LEAN) {
-        asm volatile("" : "+v"(gx));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const double gy = deriv<N, FIVE>([&](int k) { return get(X * N + k); }, Y);
+      const double gx = deriv<N, FIVE>([&](int k) { return sample(k * N + Y); }, X);
+      const double gy = deriv<N, FIVE>([&](int k) { return sample(X * N + k); }, Y);
       const double w = gauss_w<N>((X - GG::P0) * GG::M + (Y - GG::P0));
       a = a + gx * gx * w;
       b = b + gx * gy * w;
       d = d + gy * gy * w;
       if constexpr (LEAN) {
-        asm volatile("" : "+v"(a), "+v"(b), "+v"(d));
-        __builtin_amdgcn_sched_barrier(0);
+        if (POINTS || Y == GG::P1 - 1) {
+          asm volatile("" : "+v"(a), "+v"(b), "+v"(d));
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     }
   }
@@ -761,31 +765,29 @@ __device__ __forceinline__ void redecide(bool near, int o, At at, Bucket& bk) {
   }
 }
 
-// Hash of one site: FP32, re-decided in FP64 when near a boundary.  getf(i) -> float or double
-// and getd(i) -> double return window sample i (for rgb both are the FP64 luma).  LEAN picks
-// the FP64 tensor's form.
-template <int N, bool FIVE, int RULE, bool LEAN = false, typename GetF, typename GetD>
-__device__ __forceinline__ Bucket ravu_hash(GetF getf, GetD getd) {
+// Hash of one site: FP32, re-decided in FP64 when near a boundary.  get(i) returns window sample i
+// as it is stored.  LEAN picks the FP64 tensor's form.
+template <int N, bool FIVE, int RULE, bool LEAN = false, typename Get>
+__device__ __forceinline__ Bucket ravu_hash(Get get) {
   float a, b, d;
-  structure_tensor<N, FIVE>(getf, a, b, d);
+  structure_tensor<N, FIVE>(get, a, b, d);
   bool near = false;
   Bucket bk = hash_fast<RULE>(a, b, d, &near);
   if (near) {
     double ad, bd, dd;
-    structure_tensor_fp64<N, FIVE, LEAN>(getd, ad, bd, dd);
+    structure_tensor_fp64<N, FIVE, LEAN>(get, ad, bd, dd);
     bk = hash_reference<RULE, double>(ad, bd, dd);
   }
   return bk;
 }
 
-// The same with the wave's shared re-decision.  getf(i) returns
-// window sample i; o, at: see redecide.  All lanes of the wave call it together; lanes
+// The same with the wave's shared re-decision.  o, at: see redecide.  All lanes of the wave call it together; lanes
 // without a site (`valid` false) read their window too (inside the staged tile) but are never
 // re-decided.
-template <int N, bool FIVE, int RULE, int SITES, typename GetF, typename At>
-__device__ __forceinline__ Bucket ravu_hash_wave(bool valid, GetF getf, int o, At at) {
+template <int N, bool FIVE, int RULE, int SITES, typename Get, typename At>
+__device__ __forceinline__ Bucket ravu_hash_wave(bool valid, Get get, int o, At at) {
   float a, b, d;
-  structure_tensor<N, FIVE>(getf, a, b, d);
+  structure_tensor<N, FIVE>(get, a, b, d);
   bool near = false;
   Bucket bk = hash_fast<RULE>(a, b, d, &near);
   redecide<N, FIVE, RULE, SITES>(near && valid, o, at, bk);

@@ -72,7 +72,7 @@ template <int N, bool FIVE, int RULE, int CH, int PW, int PN>
 __device__ __attribute__((noinline)) Bucket redecide_site(const float* t, int o) {
   double a, b, d;
   const auto l = lds_samples(luma_plane<CH>(t, PN)) + o;
-  structure_tensor_fp64<N, FIVE, true>([&](int s) { return static_cast<double>(l[s % N * PW + s / N]); }, a, b, d);
+  structure_tensor_fp64<N, FIVE, true>([&](int s) { return l[s % N * PW + s / N]; }, a, b, d);
   return hash_reference<RULE, double>(a, b, d);
 }
 // Hash of this lane's step-1 site; all lanes of the wave together.
@@ -83,7 +83,7 @@ __device__ __forceinline__ Bucket hash_site(const float* t, int o, bool valid) {
   if constexpr (wave_redecide<CH>()) {
     return ravu_hash_wave<N, true, RULE_LOG2, kWaveSites>(valid, sample, o, [&](int at) {
       const auto w = lds_samples(l) + at;
-      return [w](int X, int Y) { return static_cast<double>(w[Y * PW + X]); };
+      return [w](int X, int Y) { return w[Y * PW + X]; };
     });
   } else {
     float a, b, d;
@@ -120,8 +120,7 @@ __global__ __launch_bounds__(TX * TY) void ravu_3x_kernel(Io io, const __half* _
   if (x >= ft.W || y >= ft.H) return;
   auto off = [&](int i) { return (ty + i % N) * PW + tx + i / N; };  // sample i = X*N + Y
   const auto* lum = luma_plane<CH>(tile, PN);
-  const Bucket bk = ravu_hash<N, false, RULE_3X>([&](int i) { return lum[off(i)]; },
-                                                 [&](int i) { return static_cast<double>(lum[off(i)]); });
+  const Bucket bk = ravu_hash<N, false, RULE_3X>([&](int i) { return lum[off(i)]; });
   const int row = bucket_row<RULE_3X>(bk, 216);
   if (io.buckets) io.buckets[f * io.bucket_bstride + static_cast<int64_t>(y) * ft.W + x] = row;
   const __half* lrow = lut + static_cast<int64_t>(row) * NTEX * 4;
@@ -312,7 +311,7 @@ struct LatticeWindow {
   static constexpr int LOW = N / 2 * (PW + 1);
   LdsSamples<T> t;
   __device__ __forceinline__ LatticeWindow(const T* lum, int at) : t(lds_samples(lum) + at - LOW) {}
-  __device__ __forceinline__ double operator()(int X, int Y) const {
+  __device__ __forceinline__ T operator()(int X, int Y) const {
     const int px = lat2x<N, STEP>(X, Y), py = lat2y<N, STEP>(X, Y);
     return t[LOW + (py >> 1) * PW + (px >> 1) + (px & 1) * NEXT];
   }
@@ -345,7 +344,7 @@ __device__ __forceinline__ void lattice_site(const Io& io, const __half* __restr
       return LatticeWindow<N, STEP, PW, NEXT, HashSample<CH>>(luma_plane<CH>(hk, PN), o);
     });
   } else {
-    bk = ravu_hash<N, true, RULE_LOG2, true>(sample, [&](int i) { return static_cast<double>(sample(i)); });
+    bk = ravu_hash<N, true, RULE_LOG2, true>(sample);
   }
   if (!valid) return;
   const int row = bucket_row<RULE_LOG2>(bk, 648);
@@ -574,7 +573,7 @@ __global__ __launch_bounds__(TX * TY / 2) __attribute__((amdgpu_waves_per_eu(4))
   auto decide = [&](int s, Bucket& bk) {
     redecide<N, true, RULE_LOG2, kWaveSites>(near[s], o, [&](int at) {
       const auto w = lds_samples(lum) + at + s * PW;
-      return [w](int X, int Y) { return static_cast<double>(w[Y * PW + X]); };
+      return [w](int X, int Y) { return w[Y * PW + X]; };
     }, bk);
     if (CH != 2 || near[s]) row[s] = bucket_row<RULE_LOG2>(bk, 648);
   };

@@ -79,8 +79,7 @@ __global__ __launch_bounds__(TX * TY) void ravu_lite_kernel(Io io, const __half*
     if constexpr (FROM_LDS) return lds(i);
     else return s[i];
   };
-  const Bucket bk = ravu_hash<N, false, RULE_LITE, FROM_LDS>(
-      [&](int i) { return sample(i); }, [&](int i) { return static_cast<double>(sample(i)); });
+  const Bucket bk = ravu_hash<N, false, RULE_LITE, FROM_LDS>(sample);
   const int row = bucket_row<RULE_LITE>(bk, 288);
   if (io.buckets)
     io.buckets[frame * io.bucket_bstride + static_cast<int64_t>(y) * ft.W + x] = row;

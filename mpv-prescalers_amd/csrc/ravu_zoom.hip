@@ -261,7 +261,7 @@ __device__ __forceinline__ void hash_bases(const HashSample<CH>* lum, int* bucke
     const Bucket bk = ravu_hash_wave<N, true, RULE_LITE, R == 2 ? 0 : kWaveSites>(
         lane_i == i, sample, by * PW + bx, [&](int o) {
           const auto t = lds_samples(lum) + o;
-          return [t](int X, int Y) { return static_cast<double>(t[Y * PW + X]); };
+          return [t](int X, int Y) { return t[Y * PW + X]; };
         });
     if (lane_i == i) bucket[by * BX + bx] = (bk.angle * 4 + bk.strength) * 3 + bk.coherence;
   }
