@@ -258,17 +258,17 @@ def serving_bench(duration_s=2.0, rate=2000.0, seed=5):
     # loop with every variant at FP32 accuracy
     single_sync = _one_per_launch(pool, reqs, prec, total_px, sync=True)
     single_async = _one_per_launch(pool, reqs, prec, total_px, sync=False)
-    plain_sync = _one_per_launch(pool, reqs, {v: "fp32" for v in prec}, total_px, sync=True)
+    fp32_sync = _one_per_launch(pool, reqs, {v: "fp32" for v in prec}, total_px, sync=True)
     small = _small_frames(prec)
     return {"workload": "Poisson %.0f frames/s, sizes %s, variants %s, 10-bit fp16 frames" %
                         (rate, "/".join("%dx%d" % s_ for s_ in SERVE_SIZES), "/".join(SERVE_VARIANTS)),
             "offered_load": offered, "saturated_mpx_s": round(sat, 1),
             "one_frame_per_launch_sync_mpx_s": round(single_sync, 1),
             "one_frame_per_launch_async_mpx_s": round(single_async, 1),
-            "one_frame_per_launch_plain_fp32_sync_mpx_s": round(plain_sync, 1),
+            "one_frame_per_launch_fp32_accuracy_sync_mpx_s": round(fp32_sync, 1),
             "speedup_vs_one_frame_per_launch_sync": round(sat / single_sync, 2),
             "speedup_vs_one_frame_per_launch_async": round(sat / single_async, 2),
-            "speedup_vs_one_frame_per_launch_plain_fp32_sync": round(sat / plain_sync, 2),
+            "speedup_vs_one_frame_per_launch_fp32_accuracy_sync": round(sat / fp32_sync, 2),
             "launches": launches, "small_frames": small,
             "native_queue": dict(native, speedup_vs_one_frame_per_launch_sync=round(native["saturated_mpx_s"] / single_sync, 2),
                                  speedup_vs_one_frame_per_launch_async=round(native["saturated_mpx_s"] / single_async, 2))}
@@ -663,9 +663,10 @@ def main():
         "config": {"workload": "nnedi3-nns32-win8x4 luma 2x, 1920x1080 fp16 plane -> 3840x2160, batch 1",
                    "variant": HEADLINE, "precision": "fp16", "in": [W, H], "out": [2 * W, 2 * H],
                    "launch": {"grid_per_cu": launch["grid_per_cu"], "split": launch["split"]}},
-        "plain_fp32": {"value": round(res["fp32"]["mpx_s"], 1), "unit": "Mpixel/s",
-                       "ms_per_step": round(res["fp32"]["ms_per_step"], 4)},
-        "speedup_vs_plain_fp32": round(f16["mpx_s"] / res["fp32"]["mpx_s"], 2),
+        "fp32_accuracy": {"value": round(res["fp32"]["mpx_s"], 1), "unit": "Mpixel/s",
+                          "ms_per_step": round(res["fp32"]["ms_per_step"], 4),
+                          "form": "three FP16 MFMA products per contraction, the kernels of fp16x3"},
+        "speedup_vs_fp32_accuracy": round(f16["mpx_s"] / res["fp32"]["mpx_s"], 2),
         "latency_ms": {"p50": round(pct(f16["times"], 50), 5), "p99": round(pct(f16["times"], 99), 5)},
         "roofline": roofline,
         "cpu_baseline": cpu,
