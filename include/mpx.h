@@ -163,8 +163,9 @@ int mpx_run_frames(mpx_plan* plan, int n, const void* const* ins, void* const* o
  * over the candidate shapes and keeps the fastest in the plan.  NNEDI3 MFMA plans: the
  * persistent grid (blocks per CU) and, for nns = 64 and 128, the neuron split across waves.
  * RAVU plans (lite, 3x, full, zoom): the tile shape of their kernels (read the choice back
- * with mpx_plan_tile); *grid_per_cu and *split are 0.  NNEDI3 FP32 plans have no tunable
- * shape: MPX_OK, nothing run.  Writes the output buffers.  Outputs (may be NULL): the
+ * with mpx_plan_tile); *grid_per_cu and *split are 0.  NNEDI3 FP32 plans keep the default
+ * shape (callers may count on it; an FP16X3 plan runs the same kernels and is tuned):
+ * MPX_OK, nothing run.  Writes the output buffers.  Outputs (may be NULL): the
  * chosen blocks per CU (0 = occupancy maximum) and split, and the best time per run in
  * microseconds.  Replaces the fixed workgroup shape of the compute shaders (e.g.
  * compute/ravu-3x-r3.hook:22 `//!COMPUTE 96 24 32 8`, compute/ravu-zoom-r3.hook:23). */
@@ -182,7 +183,7 @@ int mpx_plan_set_shape(mpx_plan* plan, int grid_per_cu, int split);
 /* Tile shape of a RAVU plan's kernels: candidate `tile` of the family's list (0 = the
  * default; mpx_plan_tune picks the fastest).  One block of the plan's kernels covers a
  * tile_w x tile_h block of input pixels (ravu-lite, ravu-3x, full RAVU) or output pixels
- * (ravu-zoom), one thread per pixel.  mpx_plan_tile outputs (may be NULL): the current
+ * (ravu-zoom), with one or two of them per thread.  mpx_plan_tile outputs (may be NULL): the current
  * index, the number of candidates (1 for NNEDI3 plans, with width = height = 0) and the
  * current tile's size.  mpx_plan_set_tile enqueues nothing and changes no result, only
  * speed; call it while no other thread runs the plan.  No counterpart in the reference

@@ -750,7 +750,7 @@ __device__ __attribute__((noinline)) Bucket redecide_alone(Sample sample) {
 // accessor (X, Y) -> sample of the window at offset o, of which `o` is this lane's.
 // Up to SITES near lanes are taken one after the other by the whole wave (wave_tensor, which also
 // says what bounds it); more evaluate their own windows at the same time.  A wave full of near
-// sites (a frame of 45-degree stripes) would take 64 turns: ravu-r4 1280x720 1512 us, against 133
+// sites (a frame of 45-degree stripes) would take 64 turns: ravu-r4 1280x720 1512 us, against 91
 // with each lane on its own.
 template <int N, bool FIVE, int RULE, int SITES, typename At>
 __device__ __forceinline__ void redecide(bool near, int o, At at, Bucket& bk) {

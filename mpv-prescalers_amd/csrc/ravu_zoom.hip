@@ -247,7 +247,8 @@ __device__ __forceinline__ const HashSample<CH>* zoom_luma(const float* tile, do
 // Hash every base pixel of a tile (nbx x nby) into bucket[by * BX + bx]: the unclamped LUT row
 // (bucket 9-row blocks are clamped per texel by the bilinear fetch, as the sampler does).
 // r2's near lanes evaluate their own windows (16 points: a turn of the wave is no cheaper, and the
-// kernel is smaller: zoom-ar-r2-rgb 4 x 720p -> 1440p 210 -> 204 us, ar-r2 134 -> 127).  TAB only
+// kernel is smaller: 4 x 720p -> 1440p zoom-ar-r2-rgb 185 -> 184 us, ar-r2 94.6 -> 92.6, large flat shapes
+// 207 -> 202, 100 -> 96).  TAB only
 // tells the kernels apart: the out-of-line evaluation follows its caller's register budget.
 template <int R, bool AR, int CH, bool TAB, int BX, int PW, int NT>
 __device__ __forceinline__ void hash_bases(const HashSample<CH>* lum, int* bucket, int nbx, int nby) {
@@ -270,7 +271,8 @@ __device__ __forceinline__ void hash_bases(const HashSample<CH>* lum, int* bucke
 // One block per TX x TY output tile, one thread per output pixel (kZoomTiles).  (Kernels
 // without anti-ringing: at least 6 waves per SIMD, a register budget their out-of-line
 // re-decision inherits; r2 anti-ringing kernels and r3 ones on 16 x 16 tiles: 5, at most 96
-// VGPRs, measured 1-8 % faster than 4 waves.)  TAB: the plan has the pre-interpolated weight table; separate instances keep the per-pixel bilinear fetch's registers out of the
+// VGPRs with 16 to 80 bytes of scratch in some, measured 1-8 % faster than 4 waves; r3-rgb misses
+// it at 108 and more.)  TAB: the plan has the pre-interpolated weight table; separate instances keep the per-pixel bilinear fetch's registers out of the
 // table path.
 template <int R, bool AR, int CH, bool TAB, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((R == 2 || TX == 16) ? 5 : 1) : 6))) void ravu_zoom_kernel(Io io, const __half* __restrict__ lut,
@@ -431,10 +433,11 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(AR ? ((
 // in_w - 1, the first and the last with one output each).  Sums run in the same order.
 // One output per thread read 1.07 KB of LDS per output for AR rgb (154 of its 287 us) beside a
 // VALU share that overlapped it badly; this form is bound by VALU issue.  4 x 720p -> 1440p,
-// one output -> two: r2 113 -> 75 us, r2-yuv 146 -> 98, r3 129 -> 101, r3-rgb 207 -> 153, ar-r2
-// 196 -> 133, ar-r2-yuv 303 -> 211, ar-r2-rgb 279 -> 211; 640 x 360 -> 1280 x 720 ar-r2 22.5 -> 19.7.
-// (r2's re-decision by each lane came after: ar-r2 126, ar-r2-rgb 204, r2-rgb 2 x 720p at 1.5x 51.)
-// 256 threads per block: 512 gave 249 us for ar-r2-rgb (waits at its two barriers), 128 gave 220.
+// one output -> two: r2 115 -> 70 us, r2-yuv 147 -> 95, r2-rgb 150 -> 97, r3 129 -> 91, r3-yuv 173 -> 120,
+// r3-rgb 207 -> 141, ar-r2 146 -> 93, ar-r2-yuv 255 -> 176, ar-r2-rgb 272 -> 184; 640 x 360 ar-r2 14.4 -> 11.9;
+// 320 x 180 within 6 % either way, 160 x 90, where half as many blocks run twice as long, up to
+// 0.8 us slower of 7.3.
+// 256 threads per block: with FP32 lumas 512 gave 249 us for ar-r2-rgb (waits at its barriers), 128 220, 256 211.
 template <int R, bool AR, int CH, int TX, int TY>
 __global__ __launch_bounds__(TX * TY) void ravu_zoom_pair_kernel(Io io, const float4* __restrict__ wtab, int nphy,
                                                                  const int4* __restrict__ phase, int out_w,
