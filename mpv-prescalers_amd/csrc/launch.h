@@ -53,11 +53,12 @@ constexpr TileShape kRavuTiles[] = {{32, 8}, {32, 16}, {64, 8}};
 constexpr TileShape kZoomTiles[] = {{32, 8}, {16, 16}};
 // Full RAVU's shapes in the order of each form, the fastest first.  luma and yuv: r3 yuv starts on
 // 64 x 8 (4 x 1080p 251.7 us, 32 x 8 264.4, 32 x 16 249.5; 640x360 20.3, 21.3, 20.4), the others on
-// 32 x 8 (r3 luma 4 x 1080p 162.0, 64 x 8 167.5, 32 x 16 173.0; r4-yuv 195.9, 205.9, 204.8).  rgb: r2 on
-// 64 x 8 (1280x720 39.8 us, 32 x 8 40.8, 32 x 16 40.6), r3 on 32 x 16 (2 x 1080p 155.4, 64 x 8 157.4, 32 x 8
-// 164.4), r4 on 32 x 8 (231.2, 32 x 16 242.9, 64 x 8 242.7).
+// 32 x 8 (r3 luma 4 x 1080p 162.0, 64 x 8 167.5, 32 x 16 173.0; r4-yuv 195.9, 205.9, 204.8).  rgb: r2 and r3
+// on 32 x 16 (r2 2 x 1080p 128.5 us, 32 x 8 129.1, 64 x 8 134.3; 1280x720 39.3, 40.2, 40.8; 640x360 19.1,
+// 19.2, 19.5; r3 159.5, 163.5, 157.1; 49.2, 50.2, 48.4; 24.1, 23.3, 23.7), r4 on 32 x 8 (230.7, 32 x 16
+// 242.6, 64 x 8 243.6).
 constexpr int ravu_tile_index(int r, int channels, int tile) {
-  const int first = channels == 2 ? (r == 2 ? 2 : r == 3 ? 1 : 0) : (channels == 1 && r == 3 ? 2 : 0);
+  const int first = channels == 2 ? (r < 4 ? 1 : 0) : (channels == 1 && r == 3 ? 2 : 0);
   return (tile + first) % 3;
 }
 constexpr int kLiteTileCount = sizeof(kLiteTiles) / sizeof(kLiteTiles[0]);
