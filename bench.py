@@ -423,10 +423,10 @@ def dominant_kernel(ctx, steps, torch):
         traffic = rec.get("hbm_bytes_per_launch")
         mfma_busy = rec.get("mfma_busy_frac")
         if rec.get("valu_instructions_per_launch"):
-            # issue model: 4 cycles per VALU instruction, 16 per transcendental, over the
+            # issue model: 4 cycles per VALU instruction, 8 per transcendental, over the
             # 1024 SIMDs at 2.4 GHz, as a share of the live kernel time
             v, t = rec["valu_instructions_per_launch"], rec["valu_transcendental_instructions_per_launch"]
-            valu_share = round(((v - t) * 4 + t * 16) / 1024 / 2.4e9 / (kms * 1e-3), 3)
+            valu_share = round(((v - t) * 4 + t * 8) / 1024 / 2.4e9 / (kms * 1e-3), 3)
     return {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_FP16, "unit": "TFLOP/s",
             "frac": round(achieved / PEAK_FP16, 4), "traffic": traffic,
             "kernel": "nnedi3_mfma double_x (fp16, nns32, win8x4)", "kernel_ms": round(kms, 5),
