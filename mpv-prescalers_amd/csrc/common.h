@@ -531,7 +531,8 @@ __device__ __forceinline__ int strength_of(T lambda) {
 
 // Eigen-analysis and bucket exactly as the reference writes it (ravu-lite-r3.hook:77-87),
 // in the reference's operation order, no contraction.  Used in FP64 for re-decisions;
-// mirrors the FP64 oracle operation for operation.
+// mirrors the FP64 oracle operation for operation; a NaN angle or strength (windows with an
+// infinity: L1 - a is inf - inf) is row 0, as there.
 template <int RULE, typename T>
 __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
 #pragma clang fp contract(off)
@@ -539,7 +540,8 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
   const T pi = T(3.141592653589793);
   T Tr = a + d;
   T D = a * d - b * b;
-  T delta = sqrt(fmax(Tr * Tr / T(4) - D, T(0)));
+  T disc = Tr * Tr / T(4) - D;
+  T delta = sqrt(disc < T(0) ? T(0) : disc);  // (fmax would drop a NaN)
   T L1 = Tr / T(2) + delta;
   T L2 = Tr / T(2) - delta;
   T sqrtL1 = sqrt(L1);
@@ -554,6 +556,7 @@ __device__ __forceinline__ Bucket hash_reference(T a, T b, T d) {
   bk.angle = static_cast<int>(floor(div_const(theta * T(24), pi, T(1) / pi)));
   bk.strength = strength_of<RULE, T>(sqrtL1);
   bk.coherence = mu >= T(0.5) ? 2 : (mu >= T(0.25) ? 1 : 0);  // NaN -> 0
+  if (theta != theta || (RULE == RULE_LOG2 && sqrtL1 != sqrtL1)) return {0, 0, 0};
   return bk;
 }
 
